@@ -2479,194 +2479,496 @@ k_beta_log(float * __restrict__ wb, long long n) {
 // ridge). The active-set loop is the reference's, step for step: the entering
 // variable is the first largest -grad over the zero set; each inner pass
 // solves the passive-set normal equations (+1e-10 on the diagonal) by
-// Gaussian elimination with partial pivoting in LDS (rows r, r + 64 in lane r),
-// interpolates back to the boundary when infeasible, and the gradient is
-// AtA w - Atb with sequential sums. Writes w (the clamp and log follow in
-// k_beta_log). Passive sets beyond LH_PMAX set *status (the host then
-// refuses the call). n <= 256: lane l owns variables l, l+64, l+128, l+192.
+// Gaussian elimination with partial pivoting, interpolates back to the
+// boundary when infeasible, and the gradient is AtA w - Atb with sequential
+// sums. Writes w (the clamp and log follow in k_beta_log). Passive sets
+// beyond LH_PMAX set *status (the host then refuses the call). n <= 256: lane
+// l owns variables l, l+64, l+128, l+192.
+//
+// What bounds it is one long dependent chain per system (an outer pass needs
+// the one before it, a pivot the update before it), so the work is cut to
+// what the results need and each pass kept short:
+//   * An outer pass is a function of (w, passive set) alone. With fewer
+//     queries than kept keys the loop soon repeats itself - a variable
+//     enters, its solve pushes it straight out again, w comes back bit for
+//     bit - and the reference repeats that pass until max_iter. A state seen
+//     before (the last two, or one saved at a power of two, Brent's method)
+//     lets the loop skip every whole period left; 32 queries and 256 keys
+//     take about 35 passes instead of 200.
+//   * The sub-problem lives in registers, one row per lane (two waves
+//     for passive sets beyond 64), shifted left by LH_SB columns every LH_SB
+//     steps so that registers are indexed statically; the row swaps are positions, not
+//     moves. Its U rows go to LDS for the back substitution, whose products
+//     are formed across the lanes and subtracted in the reference's order.
+//   * The gradient's terms with w == 0 are left out (x + 0 = x): only where
+//     every entry of AtA is finite, which its diagonal shows.
+// The 10-layer, 16-chunk, 4-head fit at n = 256 with 32 queries: 79.9 ms with
+// the sub-problem in LDS and all 200 passes, 1.6 ms now (two waves on every
+// system: 2.7 ms). 64 queries, 8 chunks: the whole call 128 -> 16.4 ms.
 // ---------------------------------------------------------------------------
-constexpr int LH_PMAX = 128;   // passive-set capacity: rows lane and lane + 64 of the sub-problem
+constexpr int LH_PMAX = 128;   // passive-set capacity
+constexpr int LH_SB = 4;       // elimination steps per rotation of the registers
 
-__global__ void __launch_bounds__(64)
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ float readlane_f(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// Two waves' offer for a step: each wave's best pivot row, from the block's
+// first column on (two sets, by the step's parity: a slower wave may still be
+// reading the step before).
+template <int W>
+struct LhOffer {
+    unsigned key, first;   // |pivot|, and the first position that has it
+    float b;
+    float row[64 * W];
+};
+
+// Step c0 + J of the elimination: pivot, the pivot row's entries from column
+// c0 on to U (at base, which moves past them) and ub, and the update of the
+// rows below. With two waves each offers the best of its rows, and both take
+// the better one from there.
+template <int W, int J>
+__device__ __forceinline__ void lh_step(float (&a)[64 * W], float & b, int & pos, int c0, int pc, float * U, float * ub,
+                                        LhOffer<W> (*of)[W], int & base, int lane, int wave) {
+    constexpr int K = 64 * W;
+    const int col = c0 + J, w = pc - c0;   // w: columns from c0 on
+    if (J >= w) return;
+    // pivot: the first row from col on of largest |a| (only strictly larger
+    // ones replace row col, NaN never does, and a NaN in row col stays)
+    const float v = fabsf(a[J]);
+    const unsigned long long dm = __ballot(pos == col);
+    int pl = dm ? __builtin_ctzll(dm) : 0, mr = col;
+    const float vd = dm ? readlane_f(v, pl) : -1.0f;
+    if (__ballot(pos > col && v > vd)) {
+        const unsigned key = (pos > col && v > vd) ? __float_as_uint(v) : 0u;
+        const unsigned km = dpp_reduce_u32<true>(key);
+        const bool cand = pos > col && v > vd && key == km;
+        const unsigned long long win = __ballot(cand);
+        if (win & (win - 1ull)) {
+            mr = (int)dpp_reduce_u32<false>(cand ? (unsigned)pos : 0xffffffffu);
+            pl = __builtin_ctzll(__ballot(pos == mr));
+        } else {
+            pl = __builtin_ctzll(win);
+            mr = __builtin_amdgcn_readlane(pos, pl);
+        }
+    }
+    float piv, pb;
+    if constexpr (W == 1) {
+        piv = readlane_f(a[J], pl);
+        pb = readlane_f(b, pl);
+        pos = lane == pl ? col : (pos == col ? mr : pos);
+        if (lane == pl) ub[col] = b;
+    } else {
+        // (a wave with no row left offers position -1 with key 0 and loses:
+        // the other wave then holds row col)
+        LhOffer<W> * o = of[J & 1];
+        const bool have = dm != 0ull || mr != col;
+        if (lane == pl) {
+            // a NaN on the diagonal stays the pivot: the largest key there is
+            o[wave].key = have ? (v == v ? __float_as_uint(v) : 0xffffffffu) : 0u;
+            o[wave].first = have ? (unsigned)mr : 0xffffffffu;
+            o[wave].b = b;
+#pragma unroll
+            for (int k0 = 0; k0 < K; k0 += 8)
+                if (k0 < w) {
+                    *reinterpret_cast<float4 *>(&o[wave].row[k0]) = make_float4(a[k0], a[k0 + 1], a[k0 + 2], a[k0 + 3]);
+                    *reinterpret_cast<float4 *>(&o[wave].row[k0 + 4]) =
+                        make_float4(a[k0 + 4], a[k0 + 5], a[k0 + 6], a[k0 + 7]);
+                }
+        }
+        __syncthreads();
+        const unsigned k0 = o[0].key, k1 = o[1].key, f0 = o[0].first, f1 = o[1].first;
+        const int best = __builtin_amdgcn_readfirstlane((k1 > k0 || (k1 == k0 && f1 < f0)) ? 1 : 0);
+        const int mrb = __builtin_amdgcn_readfirstlane((int)(best ? f1 : f0));
+        float ur[W];
+#pragma unroll
+        for (int q = 0; q < W; q++) ur[q] = o[best].row[lane + 64 * q];
+        piv = readlane_f(ur[0], J);
+        pb = o[best].b;
+        pos = pos == mrb ? col : (pos == col ? mrb : pos);
+        if (wave == best) {
+#pragma unroll
+            for (int q = 0; q < W; q++)
+                if (lane + 64 * q < w) U[base + lane + 64 * q] = ur[q];
+            if (lane == 0) ub[col] = pb;
+        }
+        base += (w + 7) & ~7;
+        if (fabsf(piv) < 1e-12f) return;
+        const float f = a[J] / piv;
+#pragma unroll
+        for (int k0 = 0; k0 < K; k0 += 8)
+            if (k0 < w) {
+#pragma unroll
+                for (int k = k0 > J ? k0 : J + 1; k < k0 + 8; k++) a[k] = a[k] - f * readlane_f(ur[k / 64], k % 64);
+            }
+        b = b - f * pb;
+        return;
+    }
+    const bool skip = fabsf(piv) < 1e-12f;
+    const float f = a[J] / piv;
+    // (rows at or above the pivot are done: what the update leaves in them is
+    // never read)
+#pragma unroll
+    for (int k0 = 0; k0 < K; k0 += 8)
+        if (k0 < w) {
+            if (lane == pl) {
+                *reinterpret_cast<float4 *>(&U[base + k0]) = make_float4(a[k0], a[k0 + 1], a[k0 + 2], a[k0 + 3]);
+                *reinterpret_cast<float4 *>(&U[base + k0 + 4]) =
+                    make_float4(a[k0 + 4], a[k0 + 5], a[k0 + 6], a[k0 + 7]);
+            }
+            if (!skip) {
+#pragma unroll
+                for (int k = k0 > J ? k0 : J + 1; k < k0 + 8; k++) a[k] = a[k] - f * readlane_f(a[k], pl);
+            }
+        }
+    if (!skip) b = b - f * pb;
+    base += (w + 7) & ~7;
+}
+
+template <int W, int... J>
+__device__ __forceinline__ void lh_steps(float (&a)[64 * W], float & b, int & pos, int c0, int pc, float * U,
+                                         float * ub, LhOffer<W> (*of)[W], int & base, int lane, int wave,
+                                         std::integer_sequence<int, J...>) {
+    (lh_step<W, J>(a, b, pos, c0, pc, U, ub, of, base, lane, wave), ...);
+}
+
+// val - p[lane 0] - p[lane 1] ... over one 16-lane row of p, in lane order
+// (each row its own: the products reach the subtraction by DPP broadcast)
+template <int... L>
+__device__ __forceinline__ float lh_chain(float val, float p, std::integer_sequence<int, L...>) {
+    ((val = val - sb_bc<L>(p)), ...);
+    return val;
+}
+
+// W = 1: passive sets of at most 64, larger ones set redo[system] and leave.
+// W = 2: every system (redo == nullptr), or those W = 1 left. The two waves
+// share the elimination (wave w holds rows 64 w .. 64 w + 63); the rest, with
+// its control flow, both compute alike.
+template <int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ? 3 : 2)))
 k_nnls_lh(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ aug,
-          const long long * __restrict__ aug_off, float * __restrict__ wout, int max_iter, int * __restrict__ status) {
+          const long long * __restrict__ aug_off, float * __restrict__ wout, int max_iter, int * __restrict__ status,
+          int * __restrict__ redo) {
+    constexpr int K = 64 * W;                       // rows and columns of the sub-problem
+    constexpr int UF = K * K / 2 + 8 * K;           // its U rows, each from its block's first column
+    static_assert(64 * 2 == LH_PMAX, "");
     const int c_idx = blockIdx.x / g.H, h = blockIdx.x % g.H, layer = blockIdx.y;
     const ChunkDesc c = chunks[c_idx];
     const int n = c.tc;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long long sys = ((long long)layer * g.n_chunks + c_idx) * g.H + h;
     float * wo = wout + ((long long)layer * g.H + h) * g.t_total + c.off;
     if (n > 256) return;   // refused on the host
-    const float * Ag = aug + aug_off[((long long)layer * g.n_chunks + c_idx) * g.H + h];
-    __shared__ float w[256], grad[256], sv[256], atb[256];
-    __shared__ unsigned char inP[256];
-    __shared__ int pidx[LH_PMAX];
-    __shared__ float sub[LH_PMAX][LH_PMAX + 2];
-    __shared__ float sP[LH_PMAX];
-    for (int i = lane; i < 256; i += 64) {
+    if (W == 2 && redo && !redo[sys]) return;
+    if (W == 1 && lane == 0) redo[sys] = 0;
+    const float * Ag = aug + aug_off[sys];
+    __shared__ __align__(16) float U[UF];
+    __shared__ float ub[K], svs[W][256], lws[W][K];
+    __shared__ int ljs[W][K];
+    __shared__ __align__(16) LhOffer<W> offer[W][W];   // (used by two waves)
+    float * sv = svs[wave], * lw = lws[wave];   // (one copy per wave: a wave may be ahead)
+    int * lj = ljs[wave];
+    float w[4], grad[4], atb[4], pw[4], p2w[4], bw[4];   // w, and the states it is compared with
+    unsigned inP = 0u, pP = 0xffffffffu, p2P = 0xffffffffu, bP = 0xffffffffu;   // bit k: variable lane + 64 k
+    bool fin = true;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = lane + 64 * k;
         const float b = i < n ? Ag[(long long)n * n + i] : 0.0f;
-        atb[i] = b;
-        w[i] = 0.0f;
-        sv[i] = 0.0f;
-        grad[i] = -b;
-        inP[i] = 0;
+        // |AtA[i][j]| and its partial sums are at most the larger diagonal entry
+        const float dg = i < n ? Ag[(long long)i * n + i] : 0.0f;
+        fin = fin && dg < 1e37f;
+        atb[k] = b;
+        w[k] = 0.0f;
+        grad[k] = -b;
+        pw[k] = p2w[k] = bw[k] = 0.0f;
     }
-    __builtin_amdgcn_wave_barrier();
-    for (int outer = 0; outer < max_iter; outer++) {
+    const bool finite = __ballot(!fin) == 0ull;
+    int lam = 0, power = 1;
+    bool cycling = false, psolved = false;   // psolved: pw is the solution of the passive set pP
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int passes = max_iter;
+    for (int outer = 0; outer < passes; outer++) {
         // entering variable: first index of the largest -grad > 0 over the zero set
         unsigned bk = 0u;
         int bi = 0x7fffffff;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const int i = lane + 64 * k;
-            if (i < n && !inP[i]) {
-                const float d = -grad[i];
-                if (d > 0.0f && __float_as_uint(d) > bk) { bk = __float_as_uint(d); bi = i; }
+            const float d = -grad[k];
+            if (i < n && !(inP >> k & 1u) && d > 0.0f && __float_as_uint(d) > bk) {
+                bk = __float_as_uint(d);
+                bi = i;
             }
         }
         const unsigned gk = dpp_reduce_u32<true>(bk);
-        const unsigned gi = dpp_reduce_u32<false>((bk == gk && bk != 0u) ? (unsigned)bi : 0xffffffffu);
+        const int t_idx = (int)dpp_reduce_u32<false>((bk == gk && bk != 0u) ? (unsigned)bi : 0xffffffffu);
         if (gk == 0u || __uint_as_float(gk) < 1e-10f) break;
-        const int t_idx = (int)gi;
-        if (lane == 0) inP[t_idx] = 1;
-        __builtin_amdgcn_wave_barrier();
+        if ((t_idx & 63) == lane) inP |= 1u << (t_idx >> 6);
+        bool solved = false;
         for (int inner = 0; inner < max_iter; inner++) {
-            // passive set, ascending
-            int pc = 0;
+            // the last pass's passive set again (the entering variable was
+            // pushed out): its solution is that pass's w
+            if (psolved && __ballot(inP != pP) == 0ull) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) w[k] = pw[k];
+                solved = true;
+                break;
+            }
+            // passive set, ascending: row r = lane + 64 q holds variable pid[q]
+            int pc = 0, rank[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const bool f = inP >> k & 1u;
+                const unsigned long long m = __ballot(f);
+                rank[k] = pc + __popcll(m & below);
+                if (f && rank[k] < K) {
+                    lj[rank[k]] = lane + 64 * k;
+                    lw[rank[k]] = atb[k];
+                }
+                pc += __popcll(m);
+            }
+            if (pc > K) {
+                if (W == 1) {
+                    if (lane == 0) redo[sys] = 1;
+                } else if (threadIdx.x == 0) {
+                    atomicOr(status, 1);
+                }
+                return;
+            }
+            wave_sync();
+            // sub-problem [AtA_PP + 1e-10 I | Atb_P]
+            unsigned pid[W];   // byte offsets
+            float a[K], b = 0.0f;
+#pragma unroll
+            for (int q = 0; q < W; q++) {
+                const int r = lane + 64 * q;
+                pid[q] = r < pc ? 4u * (unsigned)lj[r] : 0u;
+            }
+            const int row = lane + 64 * wave;
+            int pos = row < pc ? row : -1;   // logical position; -1: no row
+            if (row < pc) b = lw[row];
+            unsigned mine = pid[0];
+            if constexpr (W == 2) mine = wave ? pid[1] : pid[0];
+#pragma unroll
+            for (int k0 = 0; k0 < K; k0 += 8)
+                if (k0 < pc) {
+                    int me = row;   // opaque: K lane masks kept across the passes would spill
+                    asm volatile("" : "+v"(me));
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        const int k = k0 + u;
+                        const char * col =
+                            reinterpret_cast<const char *>(Ag) +
+                            (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)pid[k / 64], k % 64) * n;
+                        a[k] = *reinterpret_cast<const float *>(col + mine);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; u++)
+                        if (me == k0 + u) a[k0 + u] = a[k0 + u] + 1e-10f;
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 8; u++) a[k0 + u] = 0.0f;
+                }
+            // elimination, LH_SB columns at a time: in a block that starts at
+            // column c0, a[.][k] is column c0 + k
+            int base = 0;
+            for (int c0 = 0; c0 < pc; c0 += LH_SB) {
+                lh_steps<W>(a, b, pos, c0, pc, U, ub, offer, base, lane, wave,
+                            std::make_integer_sequence<int, LH_SB>());
+#pragma unroll
+                for (int k0 = 0; k0 < K; k0 += 16)
+                    if (k0 + LH_SB < pc - c0) {
+#pragma unroll
+                        for (int k = k0; k < k0 + 16 && k + LH_SB < K; k++) a[k] = a[k + LH_SB];
+                    }
+            }
+            wave_sync();
+            // back substitution: x[q] is the value of passive index lane + 64 q;
+            // the next column's entries load while one is summed
+            float x[W], un[W], pvn = 0.0f, bn = 0.0f;
+#pragma unroll
+            for (int q = 0; q < W; q++) x[q] = 0.0f;
+            auto fetch = [&](int col) {
+                const int c0 = col & ~(LH_SB - 1);
+                base -= (pc - c0 + 7) & ~7;
+#pragma unroll
+                for (int q = 0; q < W; q++) un[q] = U[base + min(max(lane + 64 * q - c0, 0), pc - c0 - 1)];
+                pvn = U[base + col - c0];
+                bn = ub[col];
+            };
+            fetch(pc - 1);
+            for (int col = pc - 1; col >= 0; col--) {
+                float prod[W], val = bn;
+                const float piv = pvn;
+#pragma unroll
+                for (int q = 0; q < W; q++) {
+                    const int r = lane + 64 * q;
+                    const float p = un[q] * x[q];
+                    prod[q] = (r > col && r < pc) ? p : 0.0f;
+                }
+                if (col > 0) fetch(col - 1);
+                if (fabsf(piv) < 1e-12f) continue;   // x stays 0
+                // in order; a product of 0 outside (col, pc) changes nothing
+#pragma unroll
+                for (int r0 = 0; r0 < K; r0 += 16)
+                    if (r0 + 15 > col && r0 < pc) {
+                        val = lh_chain(val, prod[r0 / 64], std::make_integer_sequence<int, 16>());
+                        val = readlane_f(val, r0 % 64);
+                    }
+                const float xv = val / piv;
+#pragma unroll
+                for (int q = 0; q < W; q++)
+                    if (lane + 64 * q == col) x[q] = xv;
+            }
+            bool neg = false;
+#pragma unroll
+            for (int q = 0; q < W; q++) {
+                const int r = lane + 64 * q;
+                if (r < pc) {
+                    sv[r] = x[q];
+                    neg = neg || x[q] <= 0.0f;
+                }
+            }
+            wave_sync();
+            // s over the variables (0 outside the passive set)
+            float s[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) s[k] = (inP >> k & 1u) ? sv[rank[k]] : 0.0f;
+            wave_sync();
+            if (__ballot(neg) == 0ull) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) w[k] = s[k];
+                solved = true;
+                break;
+            }
+            // step to the boundary: the smallest ratio below 1 (a minimum does
+            // not depend on the order; NaN is never taken)
+            float al = 1.0f;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if ((inP >> k & 1u) && s[k] <= 0.0f) {
+                    const float r = w[k] / (w[k] - s[k] + 1e-30f);
+                    if (r < al) al = r;
+                }
+            const unsigned ak = dpp_reduce_u32<false>(score_key(al));
+            const float alpha = __uint_as_float((ak & 0x80000000u) ? (ak & 0x7fffffffu) : ~ak);
+            bool moved = false;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const int i = lane + 64 * k;
-                const bool f = i < n && inP[i];
-                const unsigned long long m = __ballot(f);
-                const int pos = pc + __popcll(m & ((1ull << lane) - 1ull));
-                if (f && pos < LH_PMAX) pidx[pos] = i;
-                pc += __popcll(m);
-            }
-            if (pc > LH_PMAX) {
-                if (lane == 0) atomicOr(status, 1);
-                return;
-            }
-            __builtin_amdgcn_wave_barrier();
-            // sub-problem [AtA_PP + 1e-10 I | Atb_P]; rows lane and lane + 64
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const int r = lane + 64 * q;
-                if (r < pc) {
-                    const int pr = pidx[r];
-                    for (int cc = 0; cc < pc; cc++) {
-                        float v = Ag[(long long)pidx[cc] * n + pr];
-                        if (cc == r) v = v + 1e-10f;
-                        sub[r][cc] = v;
+                if (i < n) {
+                    float v = w[k] + alpha * (s[k] - w[k]);
+                    bool out = false;
+                    if ((inP >> k & 1u) && fabsf(v) < 1e-12f) {
+                        v = 0.0f;
+                        inP &= ~(1u << k);
+                        out = true;
                     }
-                    sub[r][pc] = atb[pr];
+                    moved = moved || out || __float_as_uint(v) != __float_as_uint(w[k]);
+                    w[k] = v;
                 }
             }
-            __builtin_amdgcn_wave_barrier();
-            for (int col = 0; col < pc; col++) {
-                // pivot: first row below col of largest |a| strictly above |a[col][col]|
-                const float a0 = fabsf(sub[col][col]);
-                unsigned key = 0u;
-                int kr = 0x7fffffff;
-#pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const int r = lane + 64 * q;
-                    if (r > col && r < pc) {
-                        const float v = fabsf(sub[r][col]);
-                        if (v > a0 && __float_as_uint(v) > key) { key = __float_as_uint(v); kr = r; }
-                    }
-                }
-                const unsigned km = dpp_reduce_u32<true>(key);
-                int mr = col;
-                if (km != 0u) mr = (int)dpp_reduce_u32<false>((key == km) ? (unsigned)kr : 0xffffffffu);
-                if (mr != col) {
-                    for (int j = lane; j <= pc; j += 64) {
-                        const float t0 = sub[col][j];
-                        sub[col][j] = sub[mr][j];
-                        sub[mr][j] = t0;
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();
-                const float piv = sub[col][col];
-                if (fabsf(piv) < 1e-12f) continue;
-#pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const int r = lane + 64 * q;
-                    if (r > col && r < pc) {
-                        const float f = sub[r][col] / piv;
-                        for (int j = col; j <= pc; j++) sub[r][j] = sub[r][j] - f * sub[col][j];
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
-            if (lane == 0) {
-                for (int r = 0; r < pc; r++) sP[r] = 0.0f;
-                for (int col = pc - 1; col >= 0; col--) {
-                    const float piv = sub[col][col];
-                    if (fabsf(piv) < 1e-12f) continue;
-                    float val = sub[col][pc];
-                    for (int r = col + 1; r < pc; r++) val = val - sub[col][r] * sP[r];
-                    sP[col] = val / piv;
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-            for (int i = lane; i < 256; i += 64) sv[i] = 0.0f;
-            __builtin_amdgcn_wave_barrier();
-            bool infeasible = false;
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const int r = lane + 64 * q;
-                if (r < pc) {
-                    sv[pidx[r]] = sP[r];
-                    infeasible = infeasible || (sP[r] <= 0.0f);
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (__ballot(infeasible) == 0ull) {
-                for (int i = lane; i < 256; i += 64) w[i] = sv[i];
-                __builtin_amdgcn_wave_barrier();
-                break;
-            }
-            // step to the boundary, in passive-set order
-            if (lane == 0) {
-                float alpha = 1.0f;
-                for (int r = 0; r < pc; r++) {
-                    const int idx = pidx[r];
-                    if (sv[idx] <= 0.0f) {
-                        const float a = w[idx] / (w[idx] - sv[idx] + 1e-30f);
-                        if (a < alpha) alpha = a;
-                    }
-                }
-                sP[0] = alpha;
-            }
-            __builtin_amdgcn_wave_barrier();
-            const float alpha = sP[0];
-            for (int i = lane; i < n; i += 64) w[i] = w[i] + alpha * (sv[i] - w[i]);
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const int r = lane + 64 * q;
-                if (r < pc) {
-                    const int idx = pidx[r];
-                    if (fabsf(w[idx]) < 1e-12f) {
-                        w[idx] = 0.0f;
-                        inP[idx] = 0;
-                    }
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
+            // the same state again: so would every inner pass that is left
+            if (__ballot(moved) == 0ull) break;
         }
         // grad = AtA w - Atb, sequential over j
+        int cnt = 0;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const int i = lane + 64 * k;
-            if (i < n) {
-                float sum = 0.0f;
-                for (int j = 0; j < n; j++) sum = sum + Ag[(long long)j * n + i] * w[j];
-                grad[i] = sum - atb[i];
+            const bool f = w[k] != 0.0f;   // NaN too
+            const unsigned long long m = __ballot(f);
+            const int at = cnt + __popcll(m & below);
+            if (f && at < K) {
+                lj[at] = lane + 64 * k;
+                lw[at] = w[k];
+            }
+            sv[lane + 64 * k] = w[k];
+            cnt += __popcll(m);
+        }
+        wave_sync();
+        float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        unsigned col[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) col[k] = 4u * (unsigned)min(lane + 64 * k, n - 1);
+        if (finite && cnt <= K) {
+            int jr[W];
+            float wr[W];
+#pragma unroll
+            for (int q = 0; q < W; q++) {
+                const int r = lane + 64 * q;
+                jr[q] = r < cnt ? lj[r] : 0;
+                wr[q] = r < cnt ? lw[r] : 0.0f;
+            }
+#pragma unroll
+            for (int r0 = 0; r0 < K; r0 += 8)
+                if (r0 < cnt) {
+                    float v[8][4];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        const char * row = reinterpret_cast<const char *>(
+                            Ag + (long long)__builtin_amdgcn_readlane(jr[r0 / 64], (r0 + u) % 64) * n);
+#pragma unroll
+                        for (int k = 0; k < 4; k++) v[u][k] = *reinterpret_cast<const float *>(row + col[k]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        const float wj = readlane_f(wr[r0 / 64], (r0 + u) % 64);
+#pragma unroll
+                        for (int k = 0; k < 4; k++) sum[k] = sum[k] + v[u][k] * wj;
+                    }
+                }
+        } else {
+            for (int j = 0; j < n; j++) {
+                const float wj = sv[j];
+#pragma unroll
+                for (int k = 0; k < 4; k++) sum[k] = sum[k] + Ag[(long long)j * n + col[k] / 4u] * wj;
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 4; k++) grad[k] = sum[k] - atb[k];
+        // a state met before: the passes between the two repeat to the end
+        if (!cycling) {
+            bool d1 = inP != pP, d2 = inP != p2P, db = inP != bP;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                d1 = d1 || __float_as_uint(w[k]) != __float_as_uint(pw[k]);
+                d2 = d2 || __float_as_uint(w[k]) != __float_as_uint(p2w[k]);
+                db = db || __float_as_uint(w[k]) != __float_as_uint(bw[k]);
+            }
+            lam++;
+            const int period = __ballot(d1) == 0ull ? 1 : (__ballot(d2) == 0ull ? 2 : (__ballot(db) == 0ull ? lam : 0));
+            if (period) {
+                cycling = true;
+                passes = outer + 1 + (passes - 1 - outer) % period;
+            } else if (lam == power) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) bw[k] = w[k];
+                bP = inP;
+                power *= 2;
+                lam = 0;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            p2w[k] = pw[k];
+            pw[k] = w[k];
+        }
+        p2P = pP;
+        pP = inP;
+        psolved = solved;
     }
-    for (int i = lane; i < n; i += 64) wo[i] = w[i];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = lane + 64 * k;
+        if (i < n) wo[i] = w[k];
+    }
 }
 
 // Right-hand side entry (row i, column v) of a system's [M | B] storage:
@@ -6682,8 +6984,17 @@ void launch_gather_exp(const Geom & g, const Work & w, hipStream_t st) {
 }
 
 void launch_nnls_lh(const Geom & g, const Work & w, float * wout, int max_iter, int * status, hipStream_t st) {
-    hipLaunchKernelGGL(k_nnls_lh, dim3(g.n_chunks * g.H, g.L), dim3(64), 0, st, g, w.chunks, w.aug, w.aug_off,
-                       wout, max_iter, status);
+    const dim3 grid(g.n_chunks * g.H, g.L);
+    // passive sets outgrow the query count by one or two variables, seldom
+    // more (rank and rounding), so up to 62 queries the one-wave instance goes
+    // first (32 queries, 640 systems of 256: 1.6 ms against 2.7 ms on two
+    // waves) and the other takes what it left
+    int * redo = g.nq_max <= 62 ? w.lu_redo : nullptr;
+    if (redo)
+        hipLaunchKernelGGL(k_nnls_lh<1>, grid, dim3(64), 0, st, g, w.chunks, w.aug, w.aug_off, wout, max_iter, status,
+                           redo);
+    hipLaunchKernelGGL(k_nnls_lh<2>, grid, dim3(128), 0, st, g, w.chunks, w.aug, w.aug_off, wout, max_iter, status,
+                       redo);
 }
 
 void launch_nnls_pgd(const Geom & g, const Work & w, float * wb, int iters, hipStream_t st) {
