@@ -1670,7 +1670,9 @@ k_head_sensitivity(Geom g, const ChunkDesc * __restrict__ chunks, const float * 
 // Global importance (api.cpp:656-684): max over heads (init 0, strictly
 // greater replaces), or with sensitivity weighting (math.h:605-618) the sum
 // over heads in order of sens_h * imp_h[j] from 0; then the R-KV weight.
-// grid = (n_chunks, L)
+// grid = (n_chunks, L, key blocks): a key per thread, the heads' values loaded
+// eight at a time (a state blob folds all its layers' heads into one list: 256
+// of them over 2048 keys took 730 us on the one block this was).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256)
 k_global_importance(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ imp,
@@ -1678,16 +1680,23 @@ k_global_importance(Geom g, const ChunkDesc * __restrict__ chunks, const float *
     const int c_idx = blockIdx.x, layer = blockIdx.y;
     const ChunkDesc c = chunks[c_idx];
     const float * sh = sens ? sens + ((long long)layer * g.n_chunks + c_idx) * g.H : nullptr;
-    for (int j = threadIdx.x; j < c.Tc; j += blockDim.x) {
-        float m = 0.0f;
-        for (int h = 0; h < g.H; h++) {
-            const float v = imp[((long long)layer * g.H + h) * g.T + c.start + j];
-            if (sh) m = m + sh[h] * v;
-            else if (v > m) m = v;
-        }
-        if (wts) m *= wts[c.start + j];
-        gimp[(long long)layer * g.T + c.start + j] = m;
+    const int j = blockIdx.z * 256 + threadIdx.x;
+    if (j >= c.Tc) return;
+    const float * col = imp + (long long)layer * g.H * g.T + c.start + j;
+    float m = 0.0f;
+    for (int h0 = 0; h0 < g.H; h0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = col[(long long)min(h0 + u, g.H - 1) * g.T];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (h0 + u < g.H) {
+                if (sh) m = m + sh[h0 + u] * v[u];
+                else if (v[u] > m) m = v[u];
+            }
     }
+    if (wts) m *= wts[c.start + j];
+    gimp[(long long)layer * g.T + c.start + j] = m;
 }
 
 // ---------------------------------------------------------------------------
@@ -6009,31 +6018,58 @@ k_row_softmax(float * __restrict__ x, int n, long long ls, long long hs, long lo
 
 // per (h, qi) terms in parallel (each sequential over d), then the
 // reference's accumulation order over (h, qi) on lane 0
-__global__ void __launch_bounds__(128)
+constexpr int SF_DT = 32;   // columns of the outputs staged at a time
+
+__global__ void __launch_bounds__(256)
 k_stats_final(Geom g, const float * __restrict__ oo, const float * __restrict__ co,
               int mh, int mq, float * __restrict__ stats) {
-    const int layer = blockIdx.x;
+    const int layer = blockIdx.x, tid = threadIdx.x;
+    __shared__ float ot[128][SF_DT + 1], ct[128][SF_DT + 1];
     __shared__ float t_cos[128], t_mse[128];
     __shared__ int t_agree[128];
-    const int nt = mh * mq;
-    for (int i = threadIdx.x; i < nt; i += blockDim.x) {
-        const float * o = oo + ((long long)layer * nt + i) * g.dv;
-        const float * c = co + ((long long)layer * nt + i) * g.dv;
-        float dp = 0.0f, no = 0.0f, nc = 0.0f;
-        for (int d = 0; d < g.dv; d++) { dp += o[d] * c[d]; no += o[d] * o[d]; nc += c[d] * c[d]; }
-        t_cos[i] = dp / (sqrtf(no * nc) + 1e-8f);
-        float mse = 0.0f;
-        for (int d = 0; d < g.dv; d++) { const float df = o[d] - c[d]; mse += df * df; }
-        t_mse[i] = mse / (float)g.dv;
-        int ao = 0, ac = 0;
-        for (int d = 1; d < g.dv; d++) {
-            if (o[d] > o[ao]) ao = d;
-            if (c[d] > c[ac]) ac = d;
+    const int nt = mh * mq;   // at most 4 heads x 32 queries
+    const float * o = oo + (long long)layer * nt * g.dv;
+    const float * c = co + (long long)layer * nt * g.dv;
+    // thread i owns output row i; the rows pass through LDS in slabs of
+    // columns, so that memory is read along them (one row per thread straight
+    // from memory took 70 us for 128 rows of 128, this 9)
+    float dp = 0.0f, no = 0.0f, nc = 0.0f, mse = 0.0f, mo = 0.0f, mc = 0.0f;
+    int ao = 0, ac = 0;
+    for (int d0 = 0; d0 < g.dv; d0 += SF_DT) {
+        const int dn = min(SF_DT, g.dv - d0);
+        __syncthreads();
+#pragma unroll 8
+        for (int e = tid; e < nt * SF_DT; e += 256) {
+            const int i = e / SF_DT, d = e % SF_DT;
+            const long long at = (long long)i * g.dv + d0 + min(d, dn - 1);
+            ot[i][d] = o[at];
+            ct[i][d] = c[at];
         }
-        t_agree[i] = (ao == ac) ? 1 : 0;
+        __syncthreads();
+        if (tid < nt)
+            for (int d = 0; d < dn; d++) {
+                const float x = ot[tid][d], y = ct[tid][d];
+                dp += x * y;
+                no += x * x;
+                nc += y * y;
+                const float df = x - y;
+                mse += df * df;
+                if (d0 + d == 0) {
+                    mo = x;
+                    mc = y;
+                } else {
+                    if (x > mo) { mo = x; ao = d0 + d; }
+                    if (y > mc) { mc = y; ac = d0 + d; }
+                }
+            }
+    }
+    if (tid < nt) {
+        t_cos[tid] = dp / (sqrtf(no * nc) + 1e-8f);
+        t_mse[tid] = mse / (float)g.dv;
+        t_agree[tid] = (ao == ac) ? 1 : 0;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         float sum_cos = 0.0f, sum_mse = 0.0f;
         int agree = 0;
         for (int i = 0; i < nt; i++) { sum_cos += t_cos[i]; sum_mse += t_mse[i]; agree += t_agree[i]; }
@@ -6901,7 +6937,7 @@ void launch_refit_target(const Geom & g, const Work & w, const float * V, hipStr
 }
 
 void launch_global_importance(const Geom & g, const Work & w, hipStream_t st) {
-    hipLaunchKernelGGL(k_global_importance, dim3(g.n_chunks, g.L), dim3(256), 0, st,
+    hipLaunchKernelGGL(k_global_importance, dim3(g.n_chunks, g.L, cdiv(g.Tc_max, 256)), dim3(256), 0, st,
                        g, w.chunks, w.imp, w.wts, w.sens, w.gimp);
 }
 
@@ -7219,7 +7255,7 @@ void launch_stats_compacted(const Geom & g, const Work & w, const StatWork & sw,
 }
 
 void launch_stats_final(const Geom & g, const StatWork & sw, float * stats, hipStream_t st) {
-    hipLaunchKernelGGL(k_stats_final, dim3(g.L), dim3(128), 0, st, g, sw.OO, sw.CO, sw.mh, sw.mq, stats);
+    hipLaunchKernelGGL(k_stats_final, dim3(g.L), dim3(256), 0, st, g, sw.OO, sw.CO, sw.mh, sw.mq, stats);
 }
 
 void launch_stats(const Geom & g, const Work & w, const StatWork & sw, const float * K,
