@@ -763,11 +763,11 @@ constexpr int AS_KT = 32;
 
 // Register-blocked tile: 256 threads as TQ x TV; thread (tq, tv) owns
 // queries tq + TQ*i (i < QR) and columns tv + TV*k (k < VR) of a QB x VB
-// output block (QB = TQ*QR, VB = TV*VR); every output is a sequential sum
-// over the keys in order.
+// output block (QB = TQ*QR, VB = TV*VR) from query q0 on; every output is a
+// sequential sum over the keys in order.
 template <int QR, int VR, int TV, int VC>
 __device__ __forceinline__ void attn_sum_tile(const float * __restrict__ a, const float * __restrict__ ascale,
-                                              long long a_rs, int nq,
+                                              long long a_rs, int q0, int nq,
                                               const float * __restrict__ val, long long val_rs, int n,
                                               int vn, float * __restrict__ out, long long out_rs,
                                               const RowCodec & vq, int layer, long long vrow0, int ve0) {
@@ -775,172 +775,199 @@ __device__ __forceinline__ void attn_sum_tile(const float * __restrict__ a, cons
     __shared__ float as[QB][AS_KT + 1];
     __shared__ float vs[AS_KT][VB + 1];
     const int tq = threadIdx.x / TV, tv = threadIdx.x % TV;
+    const int qb = min(QB, nq - q0);
     for (int v0 = 0; v0 < vn; v0 += VB) {
         const int vb = min(VB, vn - v0);
-        for (int q0 = 0; q0 < nq; q0 += QB) {
-            const int qb = min(QB, nq - q0);
-            float acc[QR][VR];
+        float acc[QR][VR];
+#pragma unroll
+        for (int i = 0; i < QR; i++)
+#pragma unroll
+            for (int k = 0; k < VR; k++) acc[i][k] = 0.0f;
+        for (int j0 = 0; j0 < n; j0 += AS_KT) {
+            const int jn = min(AS_KT, n - j0);
+            __syncthreads();
+            for (int e = threadIdx.x; e < QB * AS_KT; e += 256) {
+                const int qi = e / AS_KT, jj = e % AS_KT;
+                as[qi][jj] = (qi < qb && jj < jn) ? a[(long long)(q0 + qi) * a_rs + j0 + jj] * ascale[q0 + qi] : 0.0f;
+            }
+            for (int e = threadIdx.x; e < AS_KT * VB; e += 256) {
+                const int jj = e / VB, vv = e % VB;
+                // (a quantized V: token row vrow0 + j, element ve0 + column)
+                vs[jj][vv] = (jj < jn && vv < vb)
+                                 ? (VC ? codec_load1<VC>(vq, layer, vrow0 + j0 + jj, ve0 + v0 + vv)
+                                            : val[(long long)(j0 + jj) * val_rs + v0 + vv])
+                                 : 0.0f;
+            }
+            __syncthreads();
+            for (int jj = 0; jj < jn; jj++) {
+                float av[QR], vv[VR];
+#pragma unroll
+                for (int i = 0; i < QR; i++) av[i] = as[tq + TQ * i][jj];
+#pragma unroll
+                for (int k = 0; k < VR; k++) vv[k] = vs[jj][tv + TV * k];
+#pragma unroll
+                for (int i = 0; i < QR; i++)
+#pragma unroll
+                    for (int k = 0; k < VR; k++) acc[i][k] += av[i] * vv[k];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < QR; i++) {
+            const int qi = tq + TQ * i;
+#pragma unroll
+            for (int k = 0; k < VR; k++) {
+                const int vv = tv + TV * k;
+                if (qi < qb && vv < vb) out[(long long)(q0 + qi) * out_rs + v0 + vv] = acc[i][k];
+            }
+        }
+    }
+}
+
+// The same sums for a QB x VB output block (VB columns, 16-byte aligned value
+// rows) from query q0 on: thread (tq, tv) = (tid / (VB / 4), tid % (VB / 4))
+// owns queries QR tq .. QR tq + QR - 1 and columns 4 tv .. 4 tv + 3, both read
+// from LDS as one load per key; the weights are staged key-major. Tile loads
+// read rows that exist (clamped) and put zeros in registers for keys past n
+// and queries past nq, with no branch around the loads; the next tile is
+// loaded while this one is summed. A zero term leaves a sum unchanged: a sum
+// that starts at +0 never becomes -0 (x + y is -0 only when both are -0), and
+// x + (+0) = x for every other x.
+template <int VC, int VB, int QB>
+__device__ __forceinline__ void attn_sum_block(const float * __restrict__ a, const float * __restrict__ ascale,
+                                               long long a_rs, int q0, int nq,
+                                               const float * __restrict__ val, long long val_rs, int n,
+                                               float * __restrict__ out, long long out_rs,
+                                               const RowCodec & vq, int layer, long long vrow0, int ve0) {
+    constexpr int TV = VB / 4, TQ = 256 / TV, QR = QB / TQ;   // QR: 1, 2 or 4
+    constexpr int WL = QB / 32, VL = VB / 32;                 // loads per thread: weight rows, value rows
+    __shared__ __align__(16) float as[AS_KT][QB];
+    __shared__ __align__(16) float vs[AS_KT][VB];
+    const int tid = threadIdx.x, tq = tid / TV, tv = tid % TV;
+    // loaders: weights, thread -> queries lq + 32 r, keys 4 lk .. 4 lk + 3;
+    // values, thread -> keys vk + 256 / TV * u, columns 4 vc .. 4 vc + 3
+    const int lq = tid >> 3, lk = (tid & 7) * 4;
+    const int vk = tid / TV, vc = (tid % TV) * 4;
+    const float * arow[WL];
+    float sc[WL];
+#pragma unroll
+    for (int r = 0; r < WL; r++) {
+        const int q = min(q0 + lq + 32 * r, nq - 1);
+        arow[r] = a + (long long)q * a_rs;
+        sc[r] = ascale[q];
+    }
+    float ra[WL][4];
+    float4 rv[VL];
+    Raw4 rq[VL];   // (quantized V) raw value bits, decoded at the LDS store
+    // loads at clamped (valid) positions with no condition on them; the
+    // row scale and the zeros for keys past n and queries past nq are
+    // applied at the LDS store (a product or a select on a load here
+    // would make each load wait for its data before the tile is summed)
+    auto load = [&](int j0) {
+#pragma unroll
+        for (int r = 0; r < WL; r++)
+#pragma unroll
+            for (int u = 0; u < 4; u++) ra[r][u] = arow[r][min(j0 + lk + u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < VL; u++) {
+            const int j = min(j0 + vk + TQ * u, n - 1);
+            if constexpr (VC != 0) {
+                rq[u] = codec_raw4<VC>(vq, layer, vrow0 + j, ve0 + vc);
+            } else {
+                rv[u] = *reinterpret_cast<const float4 *>(val + (long long)j * val_rs + vc);
+            }
+        }
+    };
+    struct Wt { float v[QR]; };
+    auto wt = [&](int jj) {
+        Wt w;
+        if constexpr (QR == 4) {
+            const float4 x = *reinterpret_cast<const float4 *>(&as[jj][4 * tq]);
+            w.v[0] = x.x; w.v[1] = x.y; w.v[2] = x.z; w.v[3] = x.w;
+        } else if constexpr (QR == 2) {
+            const float2 x = *reinterpret_cast<const float2 *>(&as[jj][2 * tq]);
+            w.v[0] = x.x; w.v[1] = x.y;
+        } else {
+            w.v[0] = as[jj][tq];
+        }
+        return w;
+    };
+    float acc[QR][4];
+#pragma unroll
+    for (int i = 0; i < QR; i++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc[i][k] = 0.0f;
+    load(0);
+    for (int j0 = 0; j0 < n; j0 += AS_KT) {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < WL; r++)
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const float x = ra[r][u] * sc[r];
+                as[lk + u][lq + 32 * r] = (q0 + lq + 32 * r < nq && j0 + lk + u < n) ? x : 0.0f;
+            }
+#pragma unroll
+        for (int u = 0; u < VL; u++) {
+            const bool in = j0 + vk + TQ * u < n;
+            float4 x;
+            if constexpr (VC != 0) x = codec_dec4<VC>(raw_keep(in, rq[u]));
+            else x = in ? rv[u] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            *reinterpret_cast<float4 *>(&vs[vk + TQ * u][vc]) = x;
+        }
+        __syncthreads();
+        load(j0 + AS_KT);   // past the end: clamped rows, zeros (not used)
+        asm volatile("" ::: "memory");   // keeps the loads ahead of the sums
+        Wt av = wt(0);
+        float4 vv = *reinterpret_cast<const float4 *>(&vs[0][4 * tv]);
+#pragma unroll
+        for (int jj = 0; jj < AS_KT; jj++) {
+            Wt an = av;
+            float4 vn = vv;
+            if (jj + 1 < AS_KT) {
+                an = wt(jj + 1);
+                vn = *reinterpret_cast<const float4 *>(&vs[jj + 1][4 * tv]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const float vx[4] = {vv.x, vv.y, vv.z, vv.w};
 #pragma unroll
             for (int i = 0; i < QR; i++)
 #pragma unroll
-                for (int k = 0; k < VR; k++) acc[i][k] = 0.0f;
-            for (int j0 = 0; j0 < n; j0 += AS_KT) {
-                const int jn = min(AS_KT, n - j0);
-                __syncthreads();
-                for (int e = threadIdx.x; e < QB * AS_KT; e += 256) {
-                    const int qi = e / AS_KT, jj = e % AS_KT;
-                    as[qi][jj] = (qi < qb && jj < jn) ? a[(long long)(q0 + qi) * a_rs + j0 + jj] * ascale[q0 + qi] : 0.0f;
-                }
-                for (int e = threadIdx.x; e < AS_KT * VB; e += 256) {
-                    const int jj = e / VB, vv = e % VB;
-                    // (a quantized V: token row vrow0 + j, element ve0 + column)
-                    vs[jj][vv] = (jj < jn && vv < vb)
-                                     ? (VC ? codec_load1<VC>(vq, layer, vrow0 + j0 + jj, ve0 + v0 + vv)
-                                                : val[(long long)(j0 + jj) * val_rs + v0 + vv])
-                                     : 0.0f;
-                }
-                __syncthreads();
-                for (int jj = 0; jj < jn; jj++) {
-                    float av[QR], vv[VR];
-#pragma unroll
-                    for (int i = 0; i < QR; i++) av[i] = as[tq + TQ * i][jj];
-#pragma unroll
-                    for (int k = 0; k < VR; k++) vv[k] = vs[jj][tv + TV * k];
-#pragma unroll
-                    for (int i = 0; i < QR; i++)
-#pragma unroll
-                        for (int k = 0; k < VR; k++) acc[i][k] += av[i] * vv[k];
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < QR; i++) {
-                const int qi = tq + TQ * i;
-#pragma unroll
-                for (int k = 0; k < VR; k++) {
-                    const int vv = tv + TV * k;
-                    if (qi < qb && vv < vb) out[(long long)(q0 + qi) * out_rs + v0 + vv] = acc[i][k];
-                }
-            }
+                for (int k = 0; k < 4; k++) acc[i][k] = acc[i][k] + av.v[i] * vx[k];
+            __builtin_amdgcn_sched_barrier(0);
+            av = an;
+            vv = vn;
         }
+    }
+#pragma unroll
+    for (int i = 0; i < QR; i++) {
+        const int qi = q0 + QR * tq + i;
+        if (qi < nq)
+            *reinterpret_cast<float4 *>(out + (long long)qi * out_rs + 4 * tv) =
+                make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
     }
 }
 
-// The same sums for vn == 128 with 16-byte aligned value rows: a 32 x 128
-// output block, thread (tq, tv) = (tid / 32, tid % 32) owning queries
-// 4 tq .. 4 tq + 3 and columns 4 tv .. 4 tv + 3, both read from LDS as one
-// 16-byte load per key; the weights are staged key-major. Tile loads read
-// rows that exist (clamped) and put zeros in registers for keys past n and
-// queries past nq, with no branch around the loads; the next tile is loaded
-// while this one is summed. A zero term leaves a sum unchanged: a sum that
-// starts at +0 never becomes -0 (x + y is -0 only when both are -0), and
-// x + (+0) = x for every other x.
-template <int VC>
-__device__ __forceinline__ void attn_sum_128(const float * __restrict__ a, const float * __restrict__ ascale,
-                                             long long a_rs, int nq,
-                                             const float * __restrict__ val, long long val_rs, int n,
-                                             float * __restrict__ out, long long out_rs,
-                                             const RowCodec & vq, int layer, long long vrow0, int ve0) {
-    __shared__ __align__(16) float as[AS_KT][32];
-    __shared__ __align__(16) float vs[AS_KT][128];
-    const int tid = threadIdx.x, tq = tid >> 5, tv = tid & 31;
-    // loaders: weights, thread -> query lq, keys 4 lk .. 4 lk + 3;
-    // values, thread -> keys vk + 8 u, columns 4 vc .. 4 vc + 3
-    const int lq = tid >> 3, lk = (tid & 7) * 4;
-    const int vk = tid >> 5, vc = (tid & 31) * 4;
-    for (int q0 = 0; q0 < nq; q0 += 32) {
-        const bool qok = q0 + lq < nq;
-        const float * arow = a + (long long)min(q0 + lq, nq - 1) * a_rs;
-        const float sc = ascale[min(q0 + lq, nq - 1)];
-        float ra[4];
-        float4 rv[4];
-        Raw4 rq[4];   // (quantized V) raw value bits, decoded at the LDS store
-        // loads at clamped (valid) positions with no condition on them; the
-        // row scale and the zeros for keys past n and queries past nq are
-        // applied at the LDS store (a product or a select on a load here
-        // would make each load wait for its data before the tile is summed)
-        auto load = [&](int j0) {
-#pragma unroll
-            for (int u = 0; u < 4; u++) ra[u] = arow[min(j0 + lk + u, n - 1)];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int j = min(j0 + vk + 8 * u, n - 1);
-                if constexpr (VC != 0) {
-                    rq[u] = codec_raw4<VC>(vq, layer, vrow0 + j, ve0 + vc);
-                } else {
-                    rv[u] = *reinterpret_cast<const float4 *>(val + (long long)j * val_rs + vc);
-                }
-            }
-        };
-        float acc[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) acc[i][k] = 0.0f;
-        load(0);
-        for (int j0 = 0; j0 < n; j0 += AS_KT) {
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const float x = ra[u] * sc;
-                as[lk + u][lq] = (qok && j0 + lk + u < n) ? x : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const bool in = j0 + vk + 8 * u < n;
-                float4 x;
-                if constexpr (VC != 0) x = codec_dec4<VC>(raw_keep(in, rq[u]));
-                else x = in ? rv[u] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                *reinterpret_cast<float4 *>(&vs[vk + 8 * u][vc]) = x;
-            }
-            __syncthreads();
-            load(j0 + AS_KT);   // past the end: clamped rows, zeros (not used)
-            asm volatile("" ::: "memory");   // keeps the loads ahead of the sums
-            float4 av = *reinterpret_cast<const float4 *>(&as[0][4 * tq]);
-            float4 vv = *reinterpret_cast<const float4 *>(&vs[0][4 * tv]);
-#pragma unroll
-            for (int jj = 0; jj < AS_KT; jj++) {
-                float4 an = av, vn = vv;
-                if (jj + 1 < AS_KT) {
-                    an = *reinterpret_cast<const float4 *>(&as[jj + 1][4 * tq]);
-                    vn = *reinterpret_cast<const float4 *>(&vs[jj + 1][4 * tv]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                const float aa[4] = {av.x, av.y, av.z, av.w}, vx[4] = {vv.x, vv.y, vv.z, vv.w};
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-#pragma unroll
-                    for (int k = 0; k < 4; k++) acc[i][k] = acc[i][k] + aa[i] * vx[k];
-                __builtin_amdgcn_sched_barrier(0);
-                av = an;
-                vv = vn;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int qi = q0 + 4 * tq + i;
-            if (qi < nq)
-                *reinterpret_cast<float4 *>(out + (long long)qi * out_rs + 4 * tv) =
-                    make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
-        }
-    }
-}
-
-// Two kernels, so that each holds only its own LDS tiles: k_refit_target
-// for d_v = 128 with 16-byte aligned value rows (chosen on the host), and
-// k_refit_target_any for every other shape.
-template <int VC>   // 0, or the codec of a quantized V read in place (g.vc)
+// Three kernels, each output a block of its own (launch_refit_target has the
+// rule). grid (n_chunks * H, L, query blocks * column blocks):
+//   k_refit_target        QB queries x VB columns, d_v a multiple of VB with
+//                         16-byte aligned value rows;
+//   k_refit_target_any    32 queries, any d_v and alignment;
+//   k_refit_target_narrow 16 queries x 16 columns, one sum per thread, for
+//                         grids that would leave CUs idle.
+template <int VC, int VB, int QB>   // VC: 0, or the codec of a quantized V read in place (g.vc)
 __global__ void __launch_bounds__(256)
 k_refit_target(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ A,
                const float * __restrict__ ainv, const float * __restrict__ V, float * __restrict__ Y) {
     const int c_idx = blockIdx.x / g.H, h = blockIdx.x % g.H, layer = blockIdx.y;
     const ChunkDesc c = chunks[c_idx];
     const long long ev = (long long)g.H * g.dv;
-    if (c.nq <= 0 || c.Tc <= 0) return;
-    const float * sc = ainv + (((long long)layer * g.n_chunks + c_idx) * g.H + h) * g.nq_max;
-    attn_sum_128<VC>(A + layer * lS(g) + h * hS(g) + c.start, sc, g.T, c.nq,
-                 VC ? nullptr : V + layer * g.ldV + (long long)c.start * ev + (long long)h * g.dv, ev, c.Tc,
-                 Y + ((((long long)layer * g.n_chunks + c_idx) * g.H + h) * g.nq_max) * g.dv, g.dv,
-                 g.vc, layer, c.start, h * g.dv);
+    const int nv = g.dv / VB, v0 = ((int)blockIdx.z % nv) * VB, q0 = ((int)blockIdx.z / nv) * QB;
+    if (q0 >= c.nq || c.Tc <= 0) return;
+    const long long sys = ((long long)layer * g.n_chunks + c_idx) * g.H + h;
+    attn_sum_block<VC, VB, QB>(A + layer * lS(g) + h * hS(g) + c.start, ainv + sys * g.nq_max, g.T, q0, c.nq,
+                 VC ? nullptr : V + layer * g.ldV + (long long)c.start * ev + (long long)h * g.dv + v0, ev, c.Tc,
+                 Y + sys * g.nq_max * g.dv + v0, g.dv,
+                 g.vc, layer, c.start, h * g.dv + v0);
 }
 
 template <int VC>
@@ -950,12 +977,88 @@ k_refit_target_any(Geom g, const ChunkDesc * __restrict__ chunks, const float * 
     const int c_idx = blockIdx.x / g.H, h = blockIdx.x % g.H, layer = blockIdx.y;
     const ChunkDesc c = chunks[c_idx];
     const long long ev = (long long)g.H * g.dv;
-    const float * sc = ainv + (((long long)layer * g.n_chunks + c_idx) * g.H + h) * g.nq_max;
-    attn_sum_tile<4, 4, 32, VC>(A + layer * lS(g) + h * hS(g) + c.start, sc, g.T, c.nq,
+    const int q0 = (int)blockIdx.z * 32;
+    if (q0 >= c.nq) return;
+    const long long sys = ((long long)layer * g.n_chunks + c_idx) * g.H + h;
+    attn_sum_tile<4, 4, 32, VC>(A + layer * lS(g) + h * hS(g) + c.start, ainv + sys * g.nq_max, g.T, q0, c.nq,
                             VC ? nullptr : V + layer * g.ldV + (long long)c.start * ev + (long long)h * g.dv,
-                            ev, c.Tc, g.dv,
-                            Y + ((((long long)layer * g.n_chunks + c_idx) * g.H + h) * g.nq_max) * g.dv, g.dv,
+                            ev, c.Tc, g.dv, Y + sys * g.nq_max * g.dv, g.dv,
                             g.vc, layer, c.start, h * g.dv);
+}
+
+constexpr int RN_QB = 16, RN_VB = 16, RN_KT = 64;
+
+template <int VC>
+__global__ void __launch_bounds__(256)
+k_refit_target_narrow(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ A,
+                      const float * __restrict__ ainv, const float * __restrict__ V, float * __restrict__ Y) {
+    const int c_idx = blockIdx.x / g.H, h = blockIdx.x % g.H, layer = blockIdx.y;
+    const ChunkDesc c = chunks[c_idx];
+    const long long ev = (long long)g.H * g.dv;
+    const int nv = (g.dv + RN_VB - 1) / RN_VB;
+    const int v0 = ((int)blockIdx.z % nv) * RN_VB, q0 = ((int)blockIdx.z / nv) * RN_QB;
+    if (q0 >= c.nq) return;
+    const long long sys = ((long long)layer * g.n_chunks + c_idx) * g.H + h;
+    const float * a = A + layer * lS(g) + h * hS(g) + c.start;
+    const float * val = VC ? nullptr : V + layer * g.ldV + (long long)c.start * ev + (long long)h * g.dv;
+    __shared__ __align__(16) float as[2][RN_QB][RN_KT + 4];
+    __shared__ float vs[2][RN_KT][RN_VB];
+    const int n = c.Tc, tid = threadIdx.x, tq = tid >> 4, tv = tid & 15;
+    // loaders, four elements each at clamped positions: weights, thread ->
+    // query (tid >> 6) + 4 u, key tid & 63; values, thread -> key
+    // (tid >> 4) + 16 u, column tid & 15. Keys past n get weight 0 and the
+    // last key's value times 0 is not used: the sum stops at n.
+    const int kk = tid & 63, cc = min(v0 + tv, g.dv - 1);
+    const float * ar[4];
+    float sc[4], ra[4], rv[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int q = min(q0 + (tid >> 6) + 4 * u, c.nq - 1);
+        ar[u] = a + (long long)q * g.T;
+        sc[u] = ainv[sys * g.nq_max + q];
+    }
+    auto load = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) ra[u] = ar[u][min(j0 + kk, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const long long j = min(j0 + tq + 16 * u, n - 1);
+            rv[u] = VC ? codec_load1<VC>(g.vc, layer, c.start + j, h * g.dv + cc) : val[j * ev + cc];
+        }
+    };
+    auto store = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) as[b][(tid >> 6) + 4 * u][kk] = ra[u] * sc[u];
+#pragma unroll
+        for (int u = 0; u < 4; u++) vs[b][tq + 16 * u][tv] = rv[u];
+    };
+    float acc = 0.0f;
+    const int nt = (n + RN_KT - 1) / RN_KT;
+    if (nt > 0) {
+        load(0);
+        store(0);
+    }
+    __syncthreads();
+    for (int t = 0; t < nt; t++) {
+        const int b = t & 1;
+        if (t + 1 < nt) load((t + 1) * RN_KT);
+        const int jn = min(RN_KT, n - t * RN_KT);
+        if (jn == RN_KT) {
+#pragma unroll
+            for (int j4 = 0; j4 < RN_KT; j4 += 4) {
+                const float4 w = *reinterpret_cast<const float4 *>(&as[b][tq][j4]);
+                acc = acc + w.x * vs[b][j4][tv];
+                acc = acc + w.y * vs[b][j4 + 1][tv];
+                acc = acc + w.z * vs[b][j4 + 2][tv];
+                acc = acc + w.w * vs[b][j4 + 3][tv];
+            }
+        } else {
+            for (int jj = 0; jj < jn; jj++) acc = acc + as[b][tq][jj] * vs[b][jj][tv];
+        }
+        if (t + 1 < nt) store(b ^ 1);
+        __syncthreads();
+    }
+    if (q0 + tq < c.nq && v0 + tv < g.dv) Y[(sys * g.nq_max + q0 + tq) * g.dv + v0 + tv] = acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -6915,13 +7018,39 @@ void launch_chunk_softmax(const Geom & g, const Work & w, hipStream_t st) {
                            g, w.chunks, g.score_method != 0 ? w.amax : w.imp, w.sens);
 }
 
+constexpr long long RT_NARROW = 320, RT_WIDE = 1024;
+
 template <int VC>
-void launch_refit_inst(const Geom & g, const Work & w, const float * V, bool v128, hipStream_t st) {
+void launch_refit_inst(const Geom & g, const Work & w, const float * V, bool aligned, hipStream_t st) {
     const dim3 grid(g.n_chunks * g.H, g.L);
-    if (v128)
-        hipLaunchKernelGGL(k_refit_target<VC>, grid, dim3(256), 0, st, g, w.chunks, w.A, w.ainv, V, w.Y);
-    else
-        hipLaunchKernelGGL(k_refit_target_any<VC>, grid, dim3(256), 0, st, g, w.chunks, w.A, w.ainv, V, w.Y);
+    auto go = [&](auto kernel, unsigned z) {
+        hipLaunchKernelGGL(kernel, dim3(grid.x, grid.y, z), dim3(256), 0, st, g, w.chunks, w.A, w.ainv, V, w.Y);
+    };
+    // Column blocks as wide as d_v allows. Queries 64 at a time (a 64- or
+    // 32-column block then gives a thread 4 or 2 x 4 sums) where that still
+    // leaves RT_WIDE blocks, else 32. Below RT_NARROW blocks of 32 queries a
+    // block's chain over the keys is what is waited for, and one sum per
+    // thread is faster.
+    const long long units = (long long)grid.x * grid.y;
+    const int vb = g.dv % 128 == 0 ? 128 : (g.dv % 64 == 0 ? 64 : (g.dv % 32 == 0 ? 32 : 0));
+    const unsigned q32 = cdiv(g.nq_max, 32), q64 = cdiv(g.nq_max, 64);
+    if (units * q32 * (vb ? g.dv / vb : 1) < RT_NARROW) {
+        go(k_refit_target_narrow<VC>, cdiv(g.nq_max, RN_QB) * cdiv(g.dv, RN_VB));
+    } else if (!aligned || vb == 0) {
+        go(k_refit_target_any<VC>, q32);
+    } else if (vb == 128) {
+        go(k_refit_target<VC, 128, 32>, q32 * (g.dv / 128));
+    } else {
+        const unsigned nv = g.dv / vb;
+        const bool wide = g.nq_max > 32 && units * q64 * nv >= RT_WIDE;
+        if (vb == 64) {
+            if (wide) go(k_refit_target<VC, 64, 64>, q64 * nv);
+            else go(k_refit_target<VC, 64, 32>, q32 * nv);
+        } else {
+            if (wide) go(k_refit_target<VC, 32, 64>, q64 * nv);
+            else go(k_refit_target<VC, 32, 32>, q32 * nv);
+        }
+    }
 }
 
 void launch_refit_target(const Geom & g, const Work & w, const float * V, hipStream_t st) {
@@ -6929,11 +7058,10 @@ void launch_refit_target(const Geom & g, const Work & w, const float * V, hipStr
     // and the layer, token and head strides are multiples of four floats (a
     // quantized V read in place is decoded four elements at a time)
     const int vc = codec_inst(g.vc);
-    const bool v128 = g.dv == 128 && (vc || ((reinterpret_cast<uintptr_t>(V) & 15) == 0 && (g.ldV & 3) == 0 &&
-                                              (((long long)g.H * g.dv) & 3) == 0));
-    if (vc == 8) launch_refit_inst<8>(g, w, V, v128, st);
-    else if (vc == 2) launch_refit_inst<2>(g, w, V, v128, st);
-    else launch_refit_inst<0>(g, w, V, v128, st);
+    const bool aligned = g.dv % 4 == 0 && (vc || ((reinterpret_cast<uintptr_t>(V) & 15) == 0 && (g.ldV & 3) == 0));
+    if (vc == 8) launch_refit_inst<8>(g, w, V, aligned, st);
+    else if (vc == 2) launch_refit_inst<2>(g, w, V, aligned, st);
+    else launch_refit_inst<0>(g, w, V, aligned, st);
 }
 
 void launch_global_importance(const Geom & g, const Work & w, hipStream_t st) {

@@ -294,3 +294,23 @@ def test_many_reference_queries(gpu, orc):
         a = gpu.compact(K, V, Q, 3000, 300, 2, 64, 64, gpu.params(**kw))
         b = orc.compact(K, V, Q, 3000, 300, 2, 64, 64, orc.params(**kw))
         same(a, b)
+
+
+# The refit target's kernels: column blocks of 128, 64 and 32 (or none that
+# divides d_v), 32 or 64 queries a block, and the narrow form of small grids,
+# at query and key counts no block divides.
+@pytest.mark.parametrize("T,H,d,nq,chunk", [
+    (300, 1, 32, 1, -1), (300, 2, 40, 17, -1), (257, 1, 256, 33, -1), (130, 4, 64, 64, -1), (65, 1, 128, 65, -1),
+    (5135, 8, 128, 33, 128), (5135, 8, 64, 33, 128), (5135, 8, 32, 20, 128), (5135, 8, 96, 33, 128),
+    (5135, 8, 40, 33, 128), (2600, 8, 256, 20, 128), (16500, 8, 64, 65, 128), (8230, 8, 96, 65, 128)])
+def test_refit_target_blocks(gpu, orc, T, H, d, nq, chunk):
+    print(f"[refit] T={T} H={H} d={d} nq={nq} chunk={chunk}", flush=True)
+    K, V = kv_cache(T, H, d, 53, channel_scale=True)
+    Q = snapkv_queries(K, nq, 53)
+    par = dict(target_ratio=0.15, chunk_size=chunk)
+    a = gpu.compact(K, V, Q, T, nq, H, d, d, gpu.params(**par))
+    b = orc.compact(K, V, Q, T, nq, H, d, d, orc.params(**par))
+    assert np.array_equal(a.indices, b.indices), "indices"
+    assert np.array_equal(a.C_v.view(np.uint32), b.C_v.view(np.uint32)), "C_v"
+    for k in ("avg_cosine_sim", "avg_mse", "avg_agreement"):
+        assert np.float32(a.stats[k]).view(np.uint32) == np.float32(b.stats[k]).view(np.uint32), k
