@@ -5328,6 +5328,279 @@ k_ge_subst(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restri
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same substitutions for grids that would leave SIMDs idle: eight waves
+// per (system, 64 columns) instead of one, lane = column throughout. One wave
+// alone issues an instruction every 4.4 cycles, so the 65,000 terms of a
+// 256-unknown column take k_ge_subst 420 us however few systems there are
+// (128 unknowns 219 us); here 288 and 104 us, of which the forward pass is 55
+// and 21 us and the rest the backward chain, 11 cycles per subtraction
+// whether its products come from LDS or from registers.
+//   Forward: wave w owns row groups w, w + 8, .. (eight rows each) in
+// registers. When a group is finished its rows go to LDS and every wave takes
+// their eight steps off its later rows; the next group's owner does that group
+// first and finishes it in the same interval, one barrier per group.
+//   Backward: a row's sum starts with the newest value, so a column is one
+// chain of subtractions from its last row to its first. Wave 0 runs the
+// chain; waves 1..7 form the products of the next row meanwhile (wave w the
+// 4-entry blocks w - 1, w + 6, .. with those results in registers) and pass
+// them through LDS, two rows in turn, one barrier per row. They hold whole
+// solved blocks; the chain multiplies the up to four terms before the first
+// of those itself. Blocks not solved yet get products that are not read;
+// entries past n are 0 (val - 0 = val).
+// ---------------------------------------------------------------------------
+constexpr int SW_WAVES = 8, SW_HELP = SW_WAVES - 1;
+constexpr int SW_NQ = SB_NG / SW_WAVES;                     // row groups per wave of the forward pass
+constexpr int SW_NB = RG_ROWS / 4;                          // 4-entry blocks of a row
+constexpr int SW_SLOTS = (SW_NB + SW_HELP - 1) / SW_HELP;   // blocks per helper
+constexpr int SW_UR = (SW_SLOTS + 3) / 4;                   // registers of U entries per helper
+constexpr int SW_PAD = 8;                                   // zero blocks past a row's end
+constexpr int SW_LDS = 2 * (SW_NB + SW_PAD) * 64 * 4;       // floats: two rows of products (the forward's results before)
+static_assert(SW_LDS >= RG_ROWS * 64, "the forward's results fit the products' space");
+static_assert(SW_SLOTS * SW_HELP <= SW_NB + SW_PAD, "every slot has its space");
+
+// the products of a helper's slots (block SW_HELP j + hw) to the row's buffer
+template <int J>
+__device__ __forceinline__ void sw_slot(float4 * P, const float (&u)[SW_UR], const float4 (&x)[SW_SLOTS], int hw, int lane) {
+    P[(SW_HELP * J + hw) * 64 + lane] =
+        make_float4(sb_bc<4 * (J & 3)>(u[J >> 2]) * x[J].x, sb_bc<4 * (J & 3) + 1>(u[J >> 2]) * x[J].y,
+                    sb_bc<4 * (J & 3) + 2>(u[J >> 2]) * x[J].z, sb_bc<4 * (J & 3) + 3>(u[J >> 2]) * x[J].w);
+}
+// slots J0 .. J0 + 1 where they hold a block from b0 to nb - 1
+template <int J0>
+__device__ __forceinline__ void sw_pair(float4 * P, const float (&u)[SW_UR], const float4 (&x)[SW_SLOTS], int hw,
+                                        int b0, int nb, int lane) {
+    if (SW_HELP * (J0 + 1) + hw < b0 || SW_HELP * J0 + hw >= nb) return;
+    sw_slot<J0>(P, u, x, hw, lane);
+    if constexpr (J0 + 1 < SW_SLOTS) sw_slot<J0 + 1>(P, u, x, hw, lane);
+}
+template <int... K>
+__device__ __forceinline__ void sw_slots(float4 * P, const float (&u)[SW_UR], const float4 (&x)[SW_SLOTS], int hw,
+                                         int b0, int nb, int lane, std::integer_sequence<int, K...>) {
+    (sw_pair<2 * K>(P, u, x, hw, b0, nb, lane), ...);
+}
+
+// grid (systems, ceil(p / 64)), 64 * SW_WAVES threads, SW_LDS floats of dynamic LDS
+__global__ void __launch_bounds__(64 * SW_WAVES)
+k_ge_subst_wide(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ aug,
+                const long long * __restrict__ aug_off, const int * __restrict__ perm_in,
+                const unsigned char * __restrict__ skip_in, const float * __restrict__ LU_all, float * Yt_all,
+                float * __restrict__ Cv) {
+    const int sysl = blockIdx.x;   // (layer, chunk, head)
+    const int h = sysl % g.H, c_idx = (sysl / g.H) % g.n_chunks, layer = sysl / (g.H * g.n_chunks);
+    const ChunkDesc c = chunks[c_idx];
+    const int n = c.tc, p = g.dv;
+    if (n > RG_ROWS || n < 1) return;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int v = blockIdx.y * 64 + lane;
+    const bool act = v < p;
+    const int vc = act ? v : p - 1;
+    const float * __restrict__ LU = LU_all + (long long)sysl * RG_ROWS * RG_ROWS;
+    const float * __restrict__ B = aug + aug_off[sysl] + (long long)n * n;   // row-major RHS [r][v]
+    float * Yt = Yt_all + (long long)sysl * RG_ROWS * p;                     // forward results [r][v]
+    float * __restrict__ out = Cv + (((long long)layer * g.H + h) * g.t_total + c.off) * p;
+    extern __shared__ __align__(16) float sw_lds[];
+    __shared__ int permL[RG_ROWS];
+    __shared__ float ring[8][64];   // the newest results
+    bool sk = false;
+    if (tid < RG_ROWS) {
+        permL[tid] = tid < n ? perm_in[(long long)sysl * g.tc_max + tid] : 0;
+        sk = tid < n && skip_in[(long long)sysl * g.tc_max + tid] != 0;
+    }
+    if (__syncthreads_or(sk)) return;   // a skipped step: left to k_ge_solve
+    // forward
+    {
+        float (*yl)[64] = reinterpret_cast<float (*)[64]>(sw_lds);
+        float val[SW_NQ][SB_G];
+        float4 tri[SW_NQ], lb[2][SW_NQ];
+        unsigned vb[SW_NQ];
+#pragma unroll
+        for (int q = 0; q < SW_NQ; q++) {
+            const int g0 = SB_G * (wv + SW_WAVES * q);
+            // rows past n read row n - 1; nothing uses their results
+            vb[q] = (unsigned)(permL[min(g0 + ((lane & 15) >> 1), n - 1)] * RG_ROWS + 4 * (lane & 1));
+            tri[q] = sb_fload(LU, vb[q] + min(g0, RG_ROWS - SB_G));
+            lb[0][q] = sb_fload(LU, vb[q]);
+#pragma unroll
+            for (int t = 0; t < SB_G; t++) val[q][t] = B[(unsigned)(permL[min(g0 + t, n - 1)] * p + vc)];
+        }
+        auto finish = [&](int q, int gi) {
+            sb_ftri(val[q], tri[q], std::make_integer_sequence<int, SB_G>{});
+#pragma unroll
+            for (int t = 0; t < SB_G; t++) {
+                const int r = SB_G * gi + t;
+                yl[r][lane] = val[q][t];
+                if (act && r < n) Yt[(unsigned)(r * p + v)] = val[q][t];
+            }
+        };
+        if (wv == 0) finish(0, 0);
+        const int ng = (n + SB_G - 1) / SB_G;
+        // (two sets of L entries in turn, statically: a copy of a value still
+        // loading would wait for it)
+        for (int G0 = 0; G0 + 1 < ng; G0 += 2) {
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int G = G0 + k;
+                if (G + 1 >= ng) break;
+                lds_barrier();
+                float y[SB_G];
+#pragma unroll
+                for (int j = 0; j < SB_G; j++) y[j] = yl[SB_G * G + j][lane];
+#pragma unroll
+                for (int q = 0; q < SW_NQ; q++) lb[k ^ 1][q] = sb_fload(LU, vb[q] + SB_G * (G + 1));
+#pragma unroll
+                for (int q = 0; q < SW_NQ; q++)
+                    if (wv + SW_WAVES * q == G + 1) {
+                        sb_fterms(val[q], lb[k][q], y, std::make_integer_sequence<int, SB_G>{});
+                        finish(q, G + 1);
+                    }
+#pragma unroll
+                for (int q = 0; q < SW_NQ; q++)
+                    if (wv + SW_WAVES * q > G + 1 && wv + SW_WAVES * q < ng)
+                        sb_fterms(val[q], lb[k][q], y, std::make_integer_sequence<int, SB_G>{});
+            }
+        }
+    }
+    __syncthreads();
+    // backward
+    constexpr int PS = (SW_NB + SW_PAD) * 64;   // (by offset: an array of LDS pointers makes flat accesses)
+    float4 * const P = reinterpret_cast<float4 *>(sw_lds);
+    const int nb = (n + 3) / 4;
+    for (int e = tid; e < SW_PAD * 64; e += 64 * SW_WAVES) {
+        P[nb * 64 + e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        P[PS + nb * 64 + e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    __syncthreads();
+    // rows four at a time from n - 1 rounded up, so that a row's place in its
+    // block is a constant; both sides skip the rows from n on
+    const int top = (n - 1) | 3;
+    if (wv == 0) {
+        __builtin_amdgcn_s_setprio(3);   // the chain, before the helpers on its SIMD
+        // row i's entries U[i][i + d] (lane d) and its y, loaded four rows
+        // ahead; xw[d]: the result of row i + 1 + d
+        float xw[4] = {0.0f, 0.0f, 0.0f, 0.0f}, un[4], yn[4];
+        auto fetch = [&](int k, int r) {
+            r = min(max(r, 0), n - 1);
+            un[k] = LU[(unsigned)(permL[r] * RG_ROWS + r + (lane & 7))];
+            yn[k] = Yt[(unsigned)(r * p + vc)];
+        };
+#pragma unroll
+        for (int k = 0; k < 4; k++) fetch(k, top - k);
+        for (int i0 = top; i0 >= 0; i0 -= 4) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i = i0 - k;
+                const float uu = un[k];
+                float val = yn[k];
+                fetch(k, i - 4);
+                if (i >= n) continue;
+                const float piv = readlane_f(uu, 0);
+                // the terms before the first whole block of rows from i + 2 on
+                constexpr int before[4] = {4, 1, 2, 3};   // (i & 3 = 3 - k)
+#pragma unroll
+                for (int d = 0; d < 4; d++)
+                    if (d < before[k] && i + 1 + d < n) val = val - readlane_f(uu, d + 1) * xw[d];
+                int b = (i + 5) >> 2;   // the first whole block
+                if (b < nb) {
+                    const float4 * pr = P + (i & 1) * PS + lane;
+                    float4 cur[3][4];
+                    auto get = [&](int s, int at) {   // (blocks nb .. nb + 7 are zeros)
+#pragma unroll
+                        for (int m = 0; m < 4; m++) cur[s][m] = pr[(min(at, nb) + m) * 64];
+                        asm volatile("" ::: "memory");   // keeps the loads ahead of the sums
+                    };
+                    auto take = [&](int s) {
+#pragma unroll
+                        for (int m = 0; m < 4; m++) {
+                            val = val - cur[s][m].x;
+                            val = val - cur[s][m].y;
+                            val = val - cur[s][m].z;
+                            val = val - cur[s][m].w;
+                        }
+                        asm volatile("" : "+v"(val));
+                    };
+                    // four blocks summed while the next eight load
+                    get(0, b);
+                    get(1, b + 4);
+                    for (;; b += 12) {
+                        get(2, b + 8);
+                        take(0);
+                        if (b + 4 >= nb) break;
+                        get(0, b + 12);
+                        take(1);
+                        if (b + 8 >= nb) break;
+                        get(1, b + 16);
+                        take(2);
+                        if (b + 12 >= nb) break;
+                    }
+                }
+                const float xi = fabsf(piv) < 1e-12f ? g.zero_val : val / piv;
+                xw[3] = xw[2];
+                xw[2] = xw[1];
+                xw[1] = xw[0];
+                xw[0] = xi;
+                ring[i & 7][lane] = xi;
+                if (act) out[(unsigned)(i * p + v)] = xi;
+                lds_barrier();
+            }
+        }
+    } else {
+        const int hw = wv - 1;
+        float4 x[SW_SLOTS];
+#pragma unroll
+        for (int j = 0; j < SW_SLOTS; j++) x[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        // entries of the helper's blocks, four blocks per register: lane l of
+        // each 16-lane row holds entry l & 3 of block SW_HELP (4 m + (l & 15) / 4) + hw
+        int at[SW_UR];
+        bool in[SW_UR];
+#pragma unroll
+        for (int m = 0; m < SW_UR; m++) {
+            at[m] = 4 * (SW_HELP * (4 * m + ((lane & 15) >> 2)) + hw) + (lane & 3);
+            in[m] = at[m] < n;
+            at[m] = min(at[m], RG_ROWS - 1);
+        }
+        auto uload = [&](float (&u)[SW_UR], int r) {
+            r = min(max(r, 0), n - 1);
+#pragma unroll
+            for (int m = 0; m < SW_UR; m++) u[m] = LU[(unsigned)(permL[r] * RG_ROWS + at[m])];
+        };
+        float un[4][SW_UR];
+#pragma unroll
+        for (int k = 0; k < 4; k++) uload(un[k], top - k - 1);
+        // while the chain works on row i: row i - 1's products with the
+        // blocks solved by then, all entries from i + 1 on
+        for (int i0 = top; i0 >= 0; i0 -= 4) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i = i0 - k;
+                float u[SW_UR];
+#pragma unroll
+                for (int m = 0; m < SW_UR; m++) u[m] = in[m] ? un[k][m] : 0.0f;
+                uload(un[k], i - 5);
+                if (i >= n) continue;
+                const int b0 = (i + 4) >> 2;
+                if (k == 0 && b0 < nb && b0 % SW_HELP == hw) {   // block b0 has just been finished
+                    float4 w;
+                    w.x = ring[(i + 1) & 7][lane];
+                    w.y = ring[(i + 2) & 7][lane];
+                    w.z = ring[(i + 3) & 7][lane];
+                    w.w = ring[(i + 4) & 7][lane];
+                    if (4 * b0 + 1 >= n) w.y = 0.0f;
+                    if (4 * b0 + 2 >= n) w.z = 0.0f;
+                    if (4 * b0 + 3 >= n) w.w = 0.0f;
+                    const int js = b0 / SW_HELP;
+#pragma unroll
+                    for (int j = 0; j < SW_SLOTS; j++)
+                        if (j == js) x[j] = w;
+                }
+                float4 * pw = P + ((i - 1) & 1) * PS;
+                sw_slots(pw, u, x, hw, b0, nb, lane, std::make_integer_sequence<int, (SW_SLOTS + 1) / 2>());
+                lds_barrier();
+            }
+        }
+    }
+}
+
 // general size: physical row swaps in global memory, column-major storage
 __device__ void ge_solve_block(float * __restrict__ a, int n, int p, float * __restrict__ x,
                                long long ldx, float zero_val, float * prow, float * fac) {
@@ -7240,6 +7513,8 @@ void launch_ge_lu(const Geom & g, const Work & w, hipStream_t st, bool m_by_lu) 
                        g, w.chunks, w.aug, w.aug_off, X, w.perm, w.skip, w.LU, w.lu_redo, w.status, nullptr, nullptr);
 }
 
+constexpr long long SW_MAX_BLOCKS = 256;   // one per CU
+
 void launch_ge_solve(const Geom & g, const Work & w, float * Cv, hipStream_t st) {
     const unsigned systems = (unsigned)(g.L * g.n_chunks * g.H);
     // k_ge_subst solves every system without a skipped pivot step, k_ge_solve
@@ -7248,7 +7523,16 @@ void launch_ge_solve(const Geom & g, const Work & w, float * Cv, hipStream_t st)
         const char * e = getenv("KVC_SOLVE_OLD");
         return e && e[0] == '1';
     }();
-    if (!old_solve) {
+    // k_ge_subst_wide runs one block per CU: 288 us for 256 unknowns as long as
+    // every block has its CU, 580 us for 320 of them, where k_ge_subst (eight
+    // waves per CU) still takes 420 us
+    static const bool wide_ok = hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst_wide),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                    SW_LDS * (int)sizeof(float)) == hipSuccess;
+    if (!old_solve && wide_ok && (long long)systems * cdiv(g.dv, 64) <= SW_MAX_BLOCKS) {
+        hipLaunchKernelGGL(k_ge_subst_wide, dim3(systems, cdiv(g.dv, 64)), dim3(64 * SW_WAVES),
+                           SW_LDS * sizeof(float), st, g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv);
+    } else if (!old_solve) {
         const unsigned nw = cdiv(g.dv, 64);
         const size_t lds = (size_t)nw * SB_LROWS * 64 * sizeof(float);
         static int lds_ok = -1;

@@ -14,7 +14,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from kvc_data import CASE_BY_NAME, beta_variant, make_case, nonfinite_variant, nonfinite_variant_names
+from kvc_data import CASE_BY_NAME, beta_variant, kv_cache, make_case, nonfinite_variant, nonfinite_variant_names, snapkv_queries
 from kvc_harness import case_params, kc, load_oracle, run_case
 
 pytestmark = pytest.mark.gpu
@@ -85,3 +85,21 @@ def test_nonfinite_inputs(gpu, orc, name, pgd):
     a = gpu.compact(K, V, Q, T, nq, H, d, d, case_params(gpu, c, T, **extra))
     b = orc.compact(K, V, Q, T, nq, H, d, d, case_params(orc, c, T, **extra))
     same(a, b)
+
+
+# The substitution that spreads a system over eight waves (grids of at most
+# one block per CU): unknown counts around its groups of eight rows and blocks
+# of four entries, column counts around its 64 lanes.
+@pytest.mark.parametrize("n,d", [(1, 32), (2, 40), (3, 64), (4, 72), (5, 130), (8, 32), (9, 64), (31, 96), (33, 64),
+                                 (64, 256), (127, 40), (129, 64), (201, 72), (253, 64), (254, 130), (255, 64),
+                                 (256, 128)])
+def test_substitution_wide_edges(gpu, orc, n, d):
+    T = 2 * n
+    K, V = kv_cache(T, 2, d, 61, channel_scale=True)
+    nq = min(T, 24)
+    Q = snapkv_queries(K, nq, 61)
+    print(f"[subst] n={n} d={d}", flush=True)
+    a = gpu.compact(K, V, Q, T, nq, 2, d, d, gpu.params(target_ratio=0.5, chunk_size=-1))
+    b = orc.compact(K, V, Q, T, nq, 2, d, d, orc.params(target_ratio=0.5, chunk_size=-1))
+    assert a.t == b.t == n and np.array_equal(a.indices, b.indices)
+    assert np.array_equal(a.C_v.view(np.uint32), b.C_v.view(np.uint32)), "C_v"
