@@ -3109,11 +3109,16 @@ __device__ __forceinline__ long long rhs_at(int n, int p, int i, int v) {
 // over gridDim.z blocks, 512 tiles per block and pass. Rows wider than the
 // budget allows (ks < 8): one output per thread straight from global memory.
 constexpr int LB_LDS_FLOATS = 40960;   // 160 KB
-constexpr int LB_TPT = 2;              // tiles per thread and pass (slab mode)
 
-// SLAB: the instance for systems whose rows do not all fit (the launcher's
-// choice), so that the other keeps its registers
-template <bool SLAB>
+// tiles of the upper triangle of nb x nb blocks, folded into rows of nb + 1
+__host__ __device__ inline int lb_tri(int nb) { return (nb + 1) / 2 * (nb + 1); }
+
+// LB_TPT > 0: the instances for systems whose rows do not all fit (the
+// launcher's rule). A block stages every row of X and Y once per pass, so more
+// tiles per thread and pass mean less staging per sum: 512 rows of 409 + 128
+// columns, 256 systems: 5.1 ms with two tiles and the triangle's empty half
+// dealt out too, 2.7 ms with four.
+template <int LB_TPT>   // tiles per thread and pass, or 0: every system's rows fit
 __global__ void __launch_bounds__(256)
 k_ls_build(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ X,
            const float * __restrict__ Y, float * __restrict__ aug, const long long * __restrict__ aug_off,
@@ -3259,22 +3264,24 @@ k_ls_build(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restri
     // stores), or with M left to the LU only the block that also holds the
     // first columns of B; then the tiles of B alone
     const int nbm = nbi, nbr = nbw - nbm;
-    const int nmt = skip_m ? ((n & 3) ? nbi : 0) : nbi * nbm;
+    const int nmt = skip_m ? ((n & 3) ? nbi : 0) : lb_tri(nbi);
     const int njobs = nmt + nbi * nbr;
     // job -> tile (ib, jb); false: none (below the diagonal)
     auto job_tile = [&](int e, int & ib, int & jb) -> bool {
         if (e < nmt) {
             if (skip_m) { ib = e; jb = nbm - 1; return true; }
-            jb = e / nbi;
-            ib = e % nbi;
-            return ib <= jb;
+            // the triangle folded: column block nbm - 1 - q over column block q
+            const int q = e / (nbm + 1), r = e % (nbm + 1), top = nbm - q;
+            jb = r < top ? nbm - 1 - q : q;
+            ib = r < top ? r : r - top;
+            return r < top || q != nbm - 1 - q;   // (an odd count's middle column once)
         }
         e -= nmt;
         ib = e / nbr;
         jb = nbm + e % nbr;
         return true;
     };
-    if (!SLAB || whole) {
+    if (LB_TPT == 0 || whole) {
         if (blockIdx.z != 0 || !whole) return;
         stage(0, nq);
         __syncthreads();
@@ -3293,7 +3300,7 @@ k_ls_build(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restri
     }
     // slab mode: passes of LB_TPT * 256 jobs per block; every thread of the
     // block runs the same passes and slabs (the barriers are uniform)
-    if constexpr (SLAB) {
+    if constexpr (LB_TPT > 0) {
     const int per_pass = LB_TPT * (int)blockDim.x;
     for (int p0 = (int)blockIdx.z * per_pass; p0 < njobs; p0 += (int)gridDim.z * per_pass) {
         int tib[LB_TPT], tjb[LB_TPT];
@@ -7457,35 +7464,53 @@ void launch_beta_log(float * wb, long long n, hipStream_t st) {
     hipLaunchKernelGGL(k_beta_log, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, wb, n);
 }
 
+template <int TPT>
+void launch_ls_build_slab(const Geom & g, const Work & w, hipStream_t st, bool m_by_lu, int lds_floats, int nz) {
+    hipLaunchKernelGGL(k_ls_build<TPT>, dim3(g.n_chunks * g.H, g.L, nz), dim3(256), (size_t)lds_floats * sizeof(float),
+                       st, g, w.chunks, w.X, w.Y, w.aug, w.aug_off, lds_floats, m_by_lu ? 1 : 0);
+}
+
 void launch_ls_build(const Geom & g, const Work & w, hipStream_t st, bool m_by_lu) {
     // dynamic LDS beyond 64 KB needs the kernel attribute (once per process)
     static int lds_cap = -1;
-    if (lds_cap < 0)
-        lds_cap = hipFuncSetAttribute(reinterpret_cast<const void *>(k_ls_build<false>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      LB_LDS_FLOATS * (int)sizeof(float)) == hipSuccess &&
-                          hipFuncSetAttribute(reinterpret_cast<const void *>(k_ls_build<true>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              LB_LDS_FLOATS * (int)sizeof(float)) == hipSuccess
-                      ? LB_LDS_FLOATS : 16384;
+    if (lds_cap < 0) {
+        bool ok = true;
+        for (const void * k : {reinterpret_cast<const void *>(k_ls_build<0>), reinterpret_cast<const void *>(k_ls_build<1>),
+                               reinterpret_cast<const void *>(k_ls_build<2>), reinterpret_cast<const void *>(k_ls_build<4>)})
+            ok = ok && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           LB_LDS_FLOATS * (int)sizeof(float)) == hipSuccess;
+        lds_cap = ok ? LB_LDS_FLOATS : 16384;
+    }
     const long long need = (long long)g.nq_max * ((g.tc_max + g.dv + 3) & ~3);
     // every system's rows fit: one block per system; else slabs of rows
-    // through the whole budget, the tiles of a system over enough blocks to
-    // give the GPU about 2048 of them
+    // through the whole budget, the tiles of a system over several blocks
     const int wmax = (g.tc_max + g.dv + 3) & ~3;
     // (slabs of at least 8 rows in about 40 KB: four blocks per CU; whole
     // systems only up to 48 KB, three blocks per CU)
     const bool whole = need <= std::min(lds_cap, 12288);
     const int lds_floats = whole ? (int)need : std::min(lds_cap, std::max(8 * wmax, 10240));
-    const long long systems = (long long)g.n_chunks * g.H * g.L;
-    const int nz = whole ? 1 : (int)std::max<long long>(1, std::min<long long>(64, (2048 + systems - 1) / systems));
-    if (whole)
-        hipLaunchKernelGGL(k_ls_build<false>, dim3(g.n_chunks * g.H, g.L), dim3(256), (size_t)lds_floats * sizeof(float),
+    if (whole) {
+        hipLaunchKernelGGL(k_ls_build<0>, dim3(g.n_chunks * g.H, g.L), dim3(256), (size_t)lds_floats * sizeof(float),
                            st, g, w.chunks, w.X, w.Y, w.aug, w.aug_off, lds_floats, m_by_lu ? 1 : 0);
-    else
-        hipLaunchKernelGGL(k_ls_build<true>, dim3(g.n_chunks * g.H, g.L, nz), dim3(256),
-                           (size_t)lds_floats * sizeof(float), st, g, w.chunks, w.X, w.Y, w.aug, w.aug_off, lds_floats,
-                           m_by_lu ? 1 : 0);
+        return;
+    }
+    // the most tiles per thread that leave two blocks per CU (four, at three
+    // waves per SIMD, only with rows enough to sum: 32 rows of 256 + 256
+    // columns took 1.67 ms with two, 2.03 ms with four); a block takes several
+    // passes only where the systems alone give the GPU 2048 blocks
+    const long long systems = (long long)g.n_chunks * g.H * g.L;
+    const int nbi = cdiv(g.tc_max, 4), nbw = wmax / 4;
+    const bool skip_m = m_by_lu && g.tc_max <= 256;
+    const long long jobs = (skip_m ? 0 : lb_tri(nbi)) + (long long)nbi * (nbw - nbi);
+    auto passes = [&](int tpt) { return std::max<long long>(1, (jobs + 256 * tpt - 1) / (256 * tpt)); };
+    int tpt = g.nq_max >= 64 ? 4 : 2;
+    while (tpt > 1 && systems * passes(tpt) < 512) tpt /= 2;
+    const long long np = passes(tpt), zmin = (2048 + systems - 1) / systems;
+    const long long per = std::max<long long>(1, np / std::max<long long>(1, std::min(np, zmin)));
+    const int nz = (int)((np + per - 1) / per);
+    if (tpt == 4) launch_ls_build_slab<4>(g, w, st, m_by_lu, lds_floats, nz);
+    else if (tpt == 2) launch_ls_build_slab<2>(g, w, st, m_by_lu, lds_floats, nz);
+    else launch_ls_build_slab<1>(g, w, st, m_by_lu, lds_floats, nz);
 }
 
 // KVC_LU_SPLIT=0 (read at every launch) factors every system in one pass of
