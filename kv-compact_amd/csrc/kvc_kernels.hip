@@ -5686,24 +5686,20 @@ constexpr int GE_LDS_FLOATS = 8192;
 //     column of nr = n - c0 rows each). Per step c: the pivot search over
 //     column c (rows > c; the largest |a| that is not NaN, the first such row
 //     on ties, taken only when it exceeds |a[c][c]| and that is not NaN), the
-//     swap of rows c and mr in the panel, and, unless |pivot| < 1e-12 (a
-//     skipped step), the multipliers F[s][r] = a[r][c] / pivot (rows r > c)
-//     and their update of the panel's later columns. The panel's rows c0 ..
-//     c0 + pb - 1 are final and go back to memory (the rows below the
-//     diagonal are never read again).
-//  2. Trailing columns c0 + pb .. w - 1 (the rest of M, then B), each by 16
-//     lanes of one wave in an LDS column of its own: each panel step applied
-//     in order, the row swap and then, unless skipped, a[r][j] -= F[s][r] *
-//     a[c][j] for the rows r > c.
+//     swap of rows c and mr in the panel and in the earlier steps' multipliers,
+//     and, unless |pivot| < 1e-12 (a skipped step), the multipliers F[s][r] =
+//     a[r][c] / pivot (rows r > c) and their update of the panel's later
+//     columns. The panel's rows c0 .. c0 + pb - 1 are final and go back to
+//     memory (the rows below the diagonal are never read again).
+//  2. Trailing columns c0 + pb .. w - 1 (the rest of M, then B): U12 a column
+//     per thread, then a[r][j] -= F[s][r] * U12[s][j], s ascending, for the
+//     rows below in register tiles (below). Each column in LDS by 16 lanes,
+//     two LDS reads and a write per term, took the 256 systems of 409 + 128
+//     columns 8.8 ms; 5.6 ms in tiles, of which most is now the panels' serial
+//     steps and the back substitution's chain.
 // Then the back substitution of ge_solve_block. Dynamic LDS: 3 pb nr floats
-// (P, F and min(pb, blockDim.x / 16) trailing columns).
-// Order this wave's LDS accesses around the call in program order (the
-// hardware completes one wave's LDS operations in order; this keeps the
-// compiler from moving them across).
-__device__ __forceinline__ void lds_wave_order() {
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");
-}
+// (F, P and the row map, then F, U12 and the row map; nr rounded up to 4).
+constexpr int GE_PB = 32;   // widest panel
 
 __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * __restrict__ x, long long ldx,
                                  float zero_val, float * __restrict__ lds, int pb) {
@@ -5713,19 +5709,20 @@ __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * _
     __shared__ int s_mr[32];
     __shared__ unsigned char s_skip[32];
     for (int c0 = 0; c0 < n; c0 += pb) {
-        const int np = min(pb, n - c0), nr = n - c0;
-        float * P = lds;                    // P[jj * nr + (r - c0)]
-        float * F = lds + pb * nr;          // F[s * nr + (r - c0)]
-        float * Tt = lds + 2 * pb * nr;     // trailing tile, same layout as P
+        const int np = min(pb, n - c0), nr = n - c0, nrp = (nr + 3) & ~3;
+        float * F = lds;                    // multipliers F[s * nrp + (r - c0)], in the rows' final order
+        float * P = lds + pb * nrp;         // panel P[jj * nrp + (r - c0)]; later U12 in its place
+        int * src = reinterpret_cast<int *>(lds + 3 * pb * nrp - nrp);   // row that ends at c0 + r: c0 + src[r]
         __syncthreads();
         for (int e = tid; e < np * nr; e += nt) {
             const int jj = e / nr, rr = e - jj * nr;
-            P[e] = a[(long long)(c0 + jj) * n + c0 + rr];
+            P[jj * nrp + rr] = a[(long long)(c0 + jj) * n + c0 + rr];
         }
+        for (int r = tid; r < nr; r += nt) src[r] = r;
         __syncthreads();
         for (int s = 0; s < np; s++) {
             const int c = c0 + s;
-            const float * Pc = P + s * nr;
+            const float * Pc = P + s * nrp;
             // pivot search (as in ge_solve_block)
             float best = -1.0f;
             int brow = 0x7fffffff;
@@ -5751,11 +5748,17 @@ __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * _
             __syncthreads();
             const int mr = s_mr[s];
             if (mr != c) {
-                for (int jj = tid; jj < np; jj += nt) {
-                    float * col = P + jj * nr;
+                // (the earlier steps' multipliers move with their rows)
+                for (int jj = tid; jj < np + s; jj += nt) {
+                    float * col = jj < np ? P + jj * nrp : F + (jj - np) * nrp;
                     const float t0 = col[s];
                     col[s] = col[mr - c0];
                     col[mr - c0] = t0;
+                }
+                if (tid == nt - 1) {
+                    const int t0 = src[s];
+                    src[s] = src[mr - c0];
+                    src[mr - c0] = t0;
                 }
             }
             __syncthreads();
@@ -5763,13 +5766,13 @@ __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * _
             const bool skip = fabsf(piv) < 1e-12f;
             if (tid == 0) s_skip[s] = skip ? 1 : 0;
             if (!skip) {
-                for (int r = c + 1 + tid; r < n; r += nt) F[s * nr + (r - c0)] = Pc[r - c0] / piv;
+                for (int r = c + 1 + tid; r < n; r += nt) F[s * nrp + (r - c0)] = Pc[r - c0] / piv;
                 __syncthreads();
                 // 16 lanes per column, rows strided by 16
                 for (int jj = s + 1 + (tid >> 4); jj < np; jj += nt >> 4) {
-                    float * col = P + jj * nr;
+                    float * col = P + jj * nrp;
                     const float u = col[s];
-                    for (int rr = c + 1 - c0 + (tid & 15); rr < nr; rr += 16) col[rr] = col[rr] - F[s * nr + rr] * u;
+                    for (int rr = c + 1 - c0 + (tid & 15); rr < nr; rr += 16) col[rr] = col[rr] - F[s * nrp + rr] * u;
                 }
             }
             __syncthreads();
@@ -5780,40 +5783,89 @@ __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * _
         // diagonal lie contiguously at a[i n + i + 1 ..]
         for (int e = tid; e < np * np; e += nt) {
             const int jj = e / np, rr = e - jj * np;
-            a[(long long)(c0 + jj) * n + c0 + rr] = rr <= jj ? P[jj * nr + rr] : P[rr * nr + jj];
+            a[(long long)(c0 + jj) * n + c0 + rr] = rr <= jj ? P[jj * nrp + rr] : P[rr * nrp + jj];
         }
-        // trailing columns: each column by the 16 lanes of one column group
-        // (rows strided by 16) in its own LDS column; the lanes of a group
-        // are in one wave, whose LDS accesses complete in program order, so
-        // the panel's steps need no block barrier here
-        {
-            const int cg = tid >> 4, cr = tid & 15, ngr = min(nt >> 4, pb);
-            float * col = Tt + cg * nr;
-            for (int j = c0 + np + cg; cg < ngr && j < w; j += ngr) {
-                float * aj = a + (long long)j * n + c0;
-                for (int rr = cr; rr < nr; rr += 16) col[rr] = aj[rr];
-                lds_wave_order();
-                for (int s = 0; s < np; s++) {
-                    const int c = c0 + s, mr = s_mr[s];
-                    if (mr != c) {
-                        if (cr == 0) {
-                            const float t0 = col[s];
-                            col[s] = col[mr - c0];
-                            col[mr - c0] = t0;
-                        }
-                        lds_wave_order();
+        // trailing columns, as many at a time as the panel's space holds: the
+        // rows that end at c0 .. c0 + np - 1 (U12) take the panel's steps a
+        // column per thread, in registers; then every row below takes all
+        // steps in order in 4 x 4 register tiles. An element's updates are the
+        // step-by-step elimination's: a row keeps its multipliers through the
+        // swaps, and a row that ends below the panel comes from its own place
+        // or from a row of the panel (a lower row only ever moves up into the
+        // pivot row's place, for good), so rows are written in place, those of
+        // the panel last.
+        int skips = 0;
+        for (int s = 0; s < np; s++) skips |= s_skip[s];
+        const int CT = ((2 * pb - 1) * nrp / np) & ~3;
+        for (int j0 = c0 + np; j0 < w; j0 += CT) {
+            const int nc = min(CT, w - j0);
+            __syncthreads();   // the panel, or the columns before, are read
+            for (int e = tid; e < np * nc; e += nt) {
+                const int j = e / np, q = e - j * np;
+                P[q * CT + j] = a[(long long)(j0 + j) * n + c0 + src[q]];
+            }
+            __syncthreads();
+            for (int j = tid; j < nc; j += nt) {
+                float v[GE_PB];
+#pragma unroll
+                for (int q = 0; q < GE_PB; q++) v[q] = q < np ? P[q * CT + j] : 0.0f;
+#pragma unroll
+                for (int q = 0; q < GE_PB - 1; q++)
+                    if (q + 1 < np && !(skips && s_skip[q])) {
+                        const float * Fq = F + q * nrp;
+#pragma unroll
+                        for (int r = q + 1; r < GE_PB; r++)
+                            if (r < np) v[r] = v[r] - Fq[r] * v[q];
                     }
-                    if (!s_skip[s]) {
-                        const float u = col[s];
-                        const float * Fs = F + s * nr;
-                        for (int rr = c + 1 - c0 + cr; rr < nr; rr += 16) col[rr] = col[rr] - Fs[rr] * u;
-                        lds_wave_order();
-                    }
+#pragma unroll
+                for (int q = 0; q < GE_PB; q++)
+                    if (q < np) P[q * CT + j] = v[q];
+            }
+            __syncthreads();
+            const int rb = np & ~3, ntr = nr > np ? (nr - rb + 63) / 64 : 0, ntc = (nc + 15) / 16, lane = tid & 63;
+            for (int t = tid >> 6; t < ntr * ntc; t += nt >> 6) {
+                const int r0 = rb + 64 * (t % ntr) + 4 * (lane & 15), q0 = 16 * (t / ntr) + 4 * (lane >> 4);
+                const float * fp = F + min(r0, nrp - 4);
+                const float * up = P + min(q0, CT - 4);
+                float acc[4][4];
+#pragma unroll
+                for (int x = 0; x < 4; x++) {
+                    const int sr = src[min(r0 + x, nr - 1)];
+#pragma unroll
+                    for (int y = 0; y < 4; y++) acc[x][y] = a[(long long)(j0 + min(q0 + y, nc - 1)) * n + c0 + sr];
                 }
-                for (int rr = cr; rr < nr; rr += 16) aj[rr] = col[rr];
-                if (j < n)   // U rows c0 .. c0 + np - 1, transposed below the diagonal
-                    for (int rr = cr; rr < np; rr += 16) a[(long long)(c0 + rr) * n + j] = col[rr];
-                lds_wave_order();
+                float4 f = *reinterpret_cast<const float4 *>(fp), u = *reinterpret_cast<const float4 *>(up);
+                for (int q = 0; q < np; q++) {
+                    const int qn = min(q + 1, np - 1);
+                    const float4 fn = *reinterpret_cast<const float4 *>(fp + qn * nrp);
+                    const float4 un = *reinterpret_cast<const float4 *>(up + qn * CT);
+                    if (!(skips && s_skip[q])) {
+                        const float fv[4] = {f.x, f.y, f.z, f.w}, uv[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                        for (int x = 0; x < 4; x++)
+#pragma unroll
+                            for (int y = 0; y < 4; y++) acc[x][y] = acc[x][y] - fv[x] * uv[y];
+                    }
+                    f = fn;
+                    u = un;
+                }
+#pragma unroll
+                for (int y = 0; y < 4; y++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++)
+                        if (r0 + x >= np && r0 + x < nr && q0 + y < nc)
+                            a[(long long)(j0 + q0 + y) * n + c0 + r0 + x] = acc[x][y];
+            }
+            __syncthreads();
+            // U rows c0 .. c0 + np - 1 in place, and transposed below the diagonal
+            for (int e = tid; e < np * nc; e += nt) {
+                const int j = e / np, q = e - j * np;
+                a[(long long)(j0 + j) * n + c0 + q] = P[q * CT + j];
+            }
+            const int nm = min(nc, n - j0);
+            for (int e = tid; e < np * nm; e += nt) {
+                const int q = e / nm, j = e - q * nm;
+                a[(long long)(c0 + q) * n + j0 + j] = P[q * CT + j];
             }
         }
         __syncthreads();
@@ -5911,9 +5963,11 @@ __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * _
     }
 }
 
-// panel width for n rows in GE_BLK_LDS floats (3 pb n), or 0: too large
+// panel width for n rows (rounded up to 4) in GE_BLK_LDS floats (3 pb n), or
+// 0: too large
 constexpr int GE_BLK_LDS = 40960 - 256;
-__host__ __device__ inline int ge_panel(int n) { return std::min(32, GE_BLK_LDS / (3 * n)); }
+__host__ __device__ inline int ge_rows4(int n) { return (n + 3) & ~3; }
+__host__ __device__ inline int ge_panel(int n) { return std::min(GE_PB, GE_BLK_LDS / (3 * ge_rows4(n))); }
 
 __global__ void __launch_bounds__(512)
 k_ge_general(Geom g, const ChunkDesc * __restrict__ chunks, float * __restrict__ aug,
@@ -7579,7 +7633,7 @@ void launch_ge_solve(const Geom & g, const Work & w, float * Cv, hipStream_t st)
                                             hipFuncAttributeMaxDynamicSharedMemorySize,
                                             GE_BLK_LDS * (int)sizeof(float)) == hipSuccess;
         const int pb = ge_panel(g.tc_max);
-        size_t lds = pb >= 1 ? (size_t)3 * pb * g.tc_max * sizeof(float) : (size_t)GE_LDS_FLOATS * sizeof(float);
+        size_t lds = pb >= 1 ? (size_t)3 * pb * ge_rows4(g.tc_max) * sizeof(float) : (size_t)GE_LDS_FLOATS * sizeof(float);
         // without the attribute a launch above 64 KB fails, and run_batch's
         // error check turns that into -6 (the kernel is never run short of LDS)
         (void)ge_lds_ok;
