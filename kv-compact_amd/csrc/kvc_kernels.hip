@@ -626,130 +626,190 @@ __device__ __forceinline__ void lds_barrier() {
 // grid = (n_chunks * H, L)
 constexpr int SM_TILE = 64, SM_TROWS = 32;
 
+// the softmax's view of one (layer, chunk, head)
+struct SmUnit {
+    const float * Sh;   // scores, row stride rs
+    float * Ah;         // exponentials
+    long long rs;
+    int n;              // keys
+    long long ro;       // first row in ainv / rowsum
+};
+
+__device__ __forceinline__ SmUnit sm_unit(const Geom & g, const ChunkDesc & c, int c_idx, int h, int layer,
+                                          const float * S, float * A) {
+    return SmUnit{S + layer * lS(g) + h * hS(g) + c.start, A + layer * lS(g) + h * hS(g) + c.start, g.T, c.Tc,
+                  (((long long)layer * g.n_chunks + c_idx) * g.H + h) * g.nq_max};
+}
+
+// 1. maxima of rows r0 .. r0 + nr - 1 to rmax: from the scoring tiles' maxima
+//    (smax, see k_scores), or one wave per row over S
+__device__ __forceinline__ void sm_maxima(const Geom & g, const SmUnit & x, const unsigned * smax, int c_idx, int r0,
+                                          int nr, float * rmax) {
+    if (smax) {
+        const int nt = (g.Tc_max + SC_KEYS - 1) / SC_KEYS, ntc = (x.n + SC_KEYS - 1) / SC_KEYS;
+        const long long lh = x.ro / g.nq_max;   // ((layer * n_chunks + c_idx) * H + h)
+        const long long layer = lh / ((long long)g.n_chunks * g.H), h = lh % g.H;
+        for (int r = threadIdx.x; r < nr; r += blockDim.x) {
+            const unsigned * sm = smax + (((layer * g.H + h) * g.nq_max + r0 + r) * g.n_chunks + c_idx) * nt;
+            unsigned k = sm[0];
+            for (int t = 1; t < ntc; t++) k = max(k, sm[t]);
+            const float mm = __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+            const float f0 = x.Sh[(r0 + r) * x.rs];
+            rmax[r] = (f0 != f0) ? f0 : ((mm > f0) ? mm : f0);
+        }
+    } else {
+        const int lane = threadIdx.x & 63;
+        for (int r = threadIdx.x >> 6; r < nr; r += blockDim.x >> 6) {
+            const float m = wave_ref_row_max(x.Sh + (r0 + r) * x.rs, x.n, lane);
+            if (lane == 0) rmax[r] = m;
+        }
+    }
+}
+
+// 2. exponentials and ordered sums of rows r0 .. r0 + nr - 1 (nr <= TROWS);
+//    the next tile's scores load while the row sums run (barriers for LDS
+//    only). rmax: those rows' maxima; thread tid < nr returns row r0 + tid's
+//    1 / (sum + 1e-12f).
+template <int TROWS>
+__device__ __forceinline__ float sm_rows_pass(const SmUnit & x, const float * rmax, const uint64_t * etab,
+                                              float (*eb)[SM_TILE + 1], int r0, int nr, float * rowsum, float * ainv) {
+    const int tid = threadIdx.x, wv = tid >> 6, kk = tid & 63, n = x.n;
+    float sum = 0.0f;   // row r0 + tid for tid < nr
+    // this thread's rows wv, wv + 4, ... of tile t0, at clamped (in-bounds) rows and keys
+    float sv[TROWS / 4];
+    auto load = [&](int t0) {
+        const int j = t0 + min(kk, min(SM_TILE, n - t0) - 1);
+#pragma unroll
+        for (int u = 0; u < TROWS / 4; u++) sv[u] = x.Sh[(long long)(r0 + min(wv + 4 * u, nr - 1)) * x.rs + j];
+    };
+    load(0);
+    for (int t0 = 0; t0 < n; t0 += SM_TILE) {
+        const int jn = min(SM_TILE, n - t0);
+        if (kk < jn) {
+#pragma unroll
+            for (int u = 0; u < TROWS / 4; u++) {
+                const int rr = wv + 4 * u;
+                if (rr < nr) {
+                    const float e = expf_ref(sv[u] - rmax[rr], etab);
+                    eb[rr][kk] = e;
+                    x.Ah[(r0 + rr) * x.rs + t0 + kk] = e;
+                }
+            }
+        }
+        lds_barrier();
+        if (t0 + SM_TILE < n) load(t0 + SM_TILE);
+        if (tid < nr) {
+            int j = 0;
+            for (; j + 16 <= jn; j += 16) {   // 16 reads in flight, then the adds in order
+                float e[16];
+#pragma unroll
+                for (int k = 0; k < 16; k++) e[k] = eb[tid][j + k];
+#pragma unroll
+                for (int k = 0; k < 16; k++) sum += e[k];
+            }
+            for (; j < jn; j++) sum += eb[tid][j];
+        }
+        lds_barrier();
+    }
+    const float iv = 1.0f / (sum + 1e-12f);
+    if (tid < nr) {
+        if (rowsum) rowsum[x.ro + r0 + tid] = sum;
+        ainv[x.ro + r0 + tid] = iv;
+    }
+    return iv;
+}
+
+// 3. the weights of key j, aggregated in row order (rinv: 1 / (row sum + 1e-12f))
+__device__ __forceinline__ void sm_importance(const Geom & g, const SmUnit & x, const float * rinv, int nq, int j,
+                                              float * imph, float * amaxh) {
+    const float inv_m = 1.0f / (float)nq;
+    float acc = 0.0f, mx = 0.0f;
+    for (int q0 = 0; q0 < nq; q0 += 16) {
+        // sixteen rows' loads in flight, then the row-ordered aggregation
+        const int qn = min(16, nq - q0);
+        float ev[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++)
+            if (u < qn) ev[u] = x.Ah[(q0 + u) * x.rs + j];
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            if (u < qn) {
+                const float a = ev[u] * rinv[q0 + u];
+                if (g.score_method == 0) {
+                    if (a > acc) acc = a;
+                } else if (g.score_method == 1) {
+                    acc += a * a;
+                } else {
+                    acc += a;
+                }
+                if (amaxh && a > mx) mx = a;
+            }
+        }
+    }
+    if (g.score_method == 1) acc = sqrtf(acc * inv_m);
+    else if (g.score_method == 2) acc *= inv_m;
+    imph[j] = acc;
+    if (amaxh) amaxh[j] = mx;
+}
+
+// all three steps in one block per (layer, chunk, head). grid = (n_chunks * H, L)
 __global__ void __launch_bounds__(256)
 k_softmax_importance(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ S,
                      const unsigned * __restrict__ smax, float * __restrict__ A, float * __restrict__ rowsum,
                      float * __restrict__ ainv, float * __restrict__ imp, float * __restrict__ amax) {
     const int c_idx = blockIdx.x / g.H, h = blockIdx.x % g.H, layer = blockIdx.y;
     const ChunkDesc c = chunks[c_idx];
-    const long long rs = g.T;
-    const float * Sh = S + layer * lS(g) + h * hS(g) + c.start;
-    float * Ah = A + layer * lS(g) + h * hS(g) + c.start;
+    const SmUnit x = sm_unit(g, c, c_idx, h, layer, S, A);
     extern __shared__ float sm_rows[];   // row maxima, then 1 / (row sum + 1e-12f): nq_max each
     float * rmax = sm_rows;
     float * rinv = sm_rows + g.nq_max;
     __shared__ float eb[SM_TROWS][SM_TILE + 1];
     __shared__ uint64_t etab[32];
-    const int nq = c.nq, n = c.Tc;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int nq = c.nq, tid = threadIdx.x;
     if (tid < 32) etab[tid] = c_exp2_tab[tid];   // visible after the barrier below
-    // 1. row maxima: from the scoring tiles' maxima (smax, see k_scores), or
-    //    one wave per row over S
-    if (smax) {
-        const int nt = (g.Tc_max + SC_KEYS - 1) / SC_KEYS, ntc = (n + SC_KEYS - 1) / SC_KEYS;
-        for (int r = tid; r < nq; r += blockDim.x) {
-            const unsigned * sm = smax + ((((long long)layer * g.H + h) * g.nq_max + r) * g.n_chunks + c_idx) * nt;
-            unsigned k = sm[0];
-            for (int t = 1; t < ntc; t++) k = max(k, sm[t]);
-            const float mm = __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
-            const float r0 = Sh[r * rs];
-            rmax[r] = (r0 != r0) ? r0 : ((mm > r0) ? mm : r0);
-        }
-    } else {
-        for (int r = wv; r < nq; r += 4) {
-            const float m = wave_ref_row_max(Sh + r * rs, n, lane);
-            if (lane == 0) rmax[r] = m;
-        }
-    }
+    sm_maxima(g, x, smax, c_idx, 0, nq, rmax);
     __syncthreads();
-    // 2. exponentials and ordered row sums, 32 rows at a time; the next tile's
-    //    scores load while the row sums run (barriers for LDS only)
-    const int kk = tid & 63;
     for (int r0 = 0; r0 < nq; r0 += SM_TROWS) {
         const int nr = min(SM_TROWS, nq - r0);
-        float sum = 0.0f;   // row r0 + tid for tid < nr
-        // this thread's rows wv, wv + 4, ... of tile t0, at clamped (in-bounds) rows and keys
-        float sv[SM_TROWS / 4];
-        auto load = [&](int t0) {
-            const int j = t0 + min(kk, min(SM_TILE, n - t0) - 1);
-#pragma unroll
-            for (int u = 0; u < SM_TROWS / 4; u++)
-                sv[u] = Sh[(long long)(r0 + min(wv + 4 * u, nr - 1)) * rs + j];
-        };
-        load(0);
-        for (int t0 = 0; t0 < n; t0 += SM_TILE) {
-            const int jn = min(SM_TILE, n - t0);
-            if (kk < jn) {
-#pragma unroll
-                for (int u = 0; u < SM_TROWS / 4; u++) {
-                    const int rr = wv + 4 * u;
-                    if (rr < nr) {
-                        const int r = r0 + rr;
-                        const float e = expf_ref(sv[u] - rmax[r], etab);
-                        eb[rr][kk] = e;
-                        Ah[r * rs + t0 + kk] = e;
-                    }
-                }
-            }
-            lds_barrier();
-            if (t0 + SM_TILE < n) load(t0 + SM_TILE);
-            if (tid < nr) {
-                int j = 0;
-                for (; j + 16 <= jn; j += 16) {   // 16 reads in flight, then the adds in order
-                    float e[16];
-#pragma unroll
-                    for (int k = 0; k < 16; k++) e[k] = eb[tid][j + k];
-#pragma unroll
-                    for (int k = 0; k < 16; k++) sum += e[k];
-                }
-                for (; j < jn; j++) sum += eb[tid][j];
-            }
-            lds_barrier();
-        }
-        if (tid < nr) {
-            const int r = r0 + tid;
-            const long long ro = (((long long)layer * g.n_chunks + c_idx) * g.H + h) * g.nq_max + r;
-            if (rowsum) rowsum[ro] = sum;
-            const float iv = 1.0f / (sum + 1e-12f);
-            rinv[r] = iv;
-            ainv[ro] = iv;
-        }
+        const float iv = sm_rows_pass<SM_TROWS>(x, rmax + r0, etab, eb, r0, nr, rowsum, ainv);
+        if (tid < nr) rinv[r0 + tid] = iv;
     }
     __syncthreads();
-    // 3. the weights per key, aggregated in row order
-    float * imph = imp + ((long long)layer * g.H + h) * g.T + c.start;
-    const float inv_m = 1.0f / (float)nq;
-    float * amaxh = amax ? amax + ((long long)layer * g.H + h) * g.T + c.start : nullptr;
-    for (int j = tid; j < n; j += blockDim.x) {
-        float acc = 0.0f, mx = 0.0f;
-        for (int q0 = 0; q0 < nq; q0 += 16) {
-            // sixteen rows' loads in flight, then the row-ordered aggregation
-            const int qn = min(16, nq - q0);
-            float ev[16];
-#pragma unroll
-            for (int u = 0; u < 16; u++)
-                if (u < qn) ev[u] = Ah[(q0 + u) * rs + j];
-#pragma unroll
-            for (int u = 0; u < 16; u++) {
-                if (u < qn) {
-                    const int qi = q0 + u;
-                    const float a = ev[u] * rinv[qi];
-                    if (g.score_method == 0) {
-                        if (a > acc) acc = a;
-                    } else if (g.score_method == 1) {
-                        acc += a * a;
-                    } else {
-                        acc += a;
-                    }
-                    if (amaxh && a > mx) mx = a;
-                }
-            }
-        }
-        if (g.score_method == 1) acc = sqrtf(acc * inv_m);
-        else if (g.score_method == 2) acc *= inv_m;
-        imph[j] = acc;
-        if (amaxh) amaxh[j] = mx;
-    }
+    const long long io = ((long long)layer * g.H + h) * g.T + c.start;
+    for (int j = tid; j < x.n; j += blockDim.x) sm_importance(g, x, rinv, nq, j, imp + io, amax ? amax + io : nullptr);
+}
+
+// The same in two kernels, for grids that would leave CUs idle: steps 1 and 2
+// with TROWS rows a block (grid (n_chunks * H, L, row blocks)), step 3 with
+// 256 keys a block (grid (n_chunks * H, L, key blocks)).
+template <int TROWS>
+__global__ void __launch_bounds__(256)
+k_softmax_rows(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ S,
+               const unsigned * __restrict__ smax, float * __restrict__ A, float * __restrict__ rowsum,
+               float * __restrict__ ainv) {
+    const int c_idx = blockIdx.x / g.H, h = blockIdx.x % g.H, layer = blockIdx.y, r0 = (int)blockIdx.z * TROWS;
+    const ChunkDesc c = chunks[c_idx];
+    if (r0 >= c.nq) return;
+    const SmUnit x = sm_unit(g, c, c_idx, h, layer, S, A);
+    __shared__ float rmax[TROWS], eb[TROWS][SM_TILE + 1];
+    __shared__ uint64_t etab[32];
+    if (threadIdx.x < 32) etab[threadIdx.x] = c_exp2_tab[threadIdx.x];
+    const int nr = min(TROWS, c.nq - r0);
+    sm_maxima(g, x, smax, c_idx, r0, nr, rmax);
+    __syncthreads();
+    sm_rows_pass<TROWS>(x, rmax, etab, eb, r0, nr, rowsum, ainv);
+}
+
+__global__ void __launch_bounds__(256)
+k_importance(Geom g, const ChunkDesc * __restrict__ chunks, float * __restrict__ A, const float * __restrict__ ainv,
+             float * __restrict__ imp, float * __restrict__ amax) {
+    const int c_idx = blockIdx.x / g.H, h = blockIdx.x % g.H, layer = blockIdx.y;
+    const ChunkDesc c = chunks[c_idx];
+    const int j = (int)blockIdx.z * 256 + threadIdx.x;
+    if (j >= c.Tc) return;
+    const SmUnit x = sm_unit(g, c, c_idx, h, layer, nullptr, A);
+    const long long io = ((long long)layer * g.H + h) * g.T + c.start;
+    sm_importance(g, x, ainv + x.ro, c.nq, j, imp + io, amax ? amax + io : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -7340,11 +7400,27 @@ void launch_scores(const Geom & g, const ChunkDesc * chunks, int n_chunk_units, 
     }
 }
 
+constexpr long long SM_UNITS = 512;
+
 void launch_chunk_softmax(const Geom & g, const Work & w, hipStream_t st) {
-    hipLaunchKernelGGL(k_softmax_importance, dim3(g.n_chunks * g.H, g.L), dim3(256),
-                       (size_t)2 * g.nq_max * sizeof(float), st,
-                       g, w.chunks, w.S, w.smax, w.A, w.E ? w.rowsum : nullptr, w.ainv, w.imp,
-                       w.sens && g.score_method != 0 ? w.amax : nullptr);
+    float * rowsum = w.E ? w.rowsum : nullptr, * amax = w.sens && g.score_method != 0 ? w.amax : nullptr;
+    // below SM_UNITS blocks of one unit each, rows and keys over the grid: 32
+    // rows a block while that gives two blocks per CU, else 8
+    const dim3 grid(g.n_chunks * g.H, g.L);
+    const long long units = (long long)grid.x * grid.y;
+    if (units >= SM_UNITS) {
+        hipLaunchKernelGGL(k_softmax_importance, grid, dim3(256), (size_t)2 * g.nq_max * sizeof(float), st,
+                           g, w.chunks, w.S, w.smax, w.A, rowsum, w.ainv, w.imp, amax);
+    } else {
+        if (units * cdiv(g.nq_max, 32) >= 512)
+            hipLaunchKernelGGL(k_softmax_rows<32>, dim3(grid.x, grid.y, cdiv(g.nq_max, 32)), dim3(256), 0, st,
+                               g, w.chunks, w.S, w.smax, w.A, rowsum, w.ainv);
+        else
+            hipLaunchKernelGGL(k_softmax_rows<8>, dim3(grid.x, grid.y, cdiv(g.nq_max, 8)), dim3(256), 0, st,
+                               g, w.chunks, w.S, w.smax, w.A, rowsum, w.ainv);
+        hipLaunchKernelGGL(k_importance, dim3(grid.x, grid.y, cdiv(g.Tc_max, 256)), dim3(256), 0, st,
+                           g, w.chunks, w.A, w.ainv, w.imp, amax);
+    }
     // sensitivity per (layer, chunk, head) from the per-key maxima over
     // queries (the importance itself under the max score method)
     if (w.sens)
