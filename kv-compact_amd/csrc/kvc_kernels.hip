@@ -5764,7 +5764,7 @@ constexpr int GE_PB = 32;   // widest panel
 __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * __restrict__ x, long long ldx,
                                  float zero_val, float * __restrict__ lds, int pb) {
     const int w = n + p, nt = blockDim.x, tid = threadIdx.x;
-    __shared__ float bv[32];
+    __shared__ unsigned bv[32];
     __shared__ int bi[32];
     __shared__ int s_mr[32];
     __shared__ unsigned char s_skip[32];
@@ -5783,8 +5783,10 @@ __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * _
         for (int s = 0; s < np; s++) {
             const int c = c0 + s;
             const float * Pc = P + s * nrp;
-            // pivot search (as in ge_solve_block)
-            float best = -1.0f;
+            // pivot search: the first largest |a| above row c's that is not
+            // NaN, per wave, then over the waves by every wave alike
+            const float a0 = fabsf(Pc[s]);
+            unsigned bk = 0u;
             int brow = 0x7fffffff;
             for (int r = c + 1 + tid; r < n; r += nt) {
                 const float v = fabsf(Pc[r - c0]);
@@ -5832,7 +5834,20 @@ __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * _
                 for (int jj = s + 1 + (tid >> 4); jj < np; jj += nt >> 4) {
                     float * col = P + jj * nrp;
                     const float u = col[s];
-                    for (int rr = c + 1 - c0 + (tid & 15); rr < nr; rr += 16) col[rr] = col[rr] - F[s * nrp + rr] * u;
+                    // eight rows' reads in flight before their writes
+                    const float * Fs = F + s * nrp;
+                    for (int rr = c + 1 - c0 + (tid & 15); rr < nr; rr += 128) {
+                        float x[8], m[8];
+#pragma unroll
+                        for (int k = 0; k < 8; k++) {
+                            const int q = min(rr + 16 * k, nr - 1);
+                            x[k] = col[q];
+                            m[k] = Fs[q];
+                        }
+#pragma unroll
+                        for (int k = 0; k < 8; k++)
+                            if (rr + 16 * k < nr) col[rr + 16 * k] = x[k] - m[k] * u;
+                    }
                 }
             }
             __syncthreads();
