@@ -5447,19 +5447,39 @@ __device__ __forceinline__ void sw_slots(float4 * P, const float (&u)[SW_UR], co
     (sw_pair<2 * K>(P, u, x, hw, b0, nb, lane), ...);
 }
 
-// grid (systems, ceil(p / 64)), 64 * SW_WAVES threads, SW_LDS floats of dynamic LDS
-__global__ void __launch_bounds__(64 * SW_WAVES)
-k_ge_subst_wide(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ aug,
-                const long long * __restrict__ aug_off, const int * __restrict__ perm_in,
-                const unsigned char * __restrict__ skip_in, const float * __restrict__ LU_all, float * Yt_all,
-                float * __restrict__ Cv) {
-    const int sysl = blockIdx.x;   // (layer, chunk, head)
+// the forward terms of one group's eight steps, without the skipped ones (bit
+// J of mask): the reference leaves out a skipped step's elimination
+template <int... J>
+__device__ __forceinline__ void sw_fterms(float (&val)[SB_G], const float4 & b, const float * y, unsigned mask,
+                                          std::integer_sequence<int, J...>) {
+    ((mask >> J & 1u ? (void)0 : sb_fstep<J>(val, b, y[J], std::make_integer_sequence<int, SB_G>{})), ...);
+}
+template <int T, int... R>
+__device__ __forceinline__ void sw_ftri_row(float (&val)[SB_G], const float4 & b, unsigned mask,
+                                            std::integer_sequence<int, R...>) {
+    ((val[T] = mask >> R & 1u ? val[T] : val[T] - sb_fl<R, T>(b) * val[R]), ...);
+}
+template <int... T>
+__device__ __forceinline__ void sw_ftri(float (&val)[SB_G], const float4 & b, unsigned mask,
+                                        std::integer_sequence<int, T...>) {
+    (sw_ftri_row<T>(val, b, mask, std::make_integer_sequence<int, T>{}), ...);
+}
+
+// one system (layer, chunk, head) and 64 columns. SKIP: systems with skipped
+// steps, else those without (the others return at once)
+template <bool SKIP>
+__device__ __forceinline__ void subst_wide(const Geom & g, const ChunkDesc * __restrict__ chunks,
+                                           const float * __restrict__ aug, const long long * __restrict__ aug_off,
+                                           const int * __restrict__ perm_in,
+                                           const unsigned char * __restrict__ skip_in,
+                                           const float * __restrict__ LU_all, float * Yt_all, float * __restrict__ Cv,
+                                           int sysl, int vblock) {
     const int h = sysl % g.H, c_idx = (sysl / g.H) % g.n_chunks, layer = sysl / (g.H * g.n_chunks);
     const ChunkDesc c = chunks[c_idx];
     const int n = c.tc, p = g.dv;
     if (n > RG_ROWS || n < 1) return;
     const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int v = blockIdx.y * 64 + lane;
+    const int v = vblock * 64 + lane;
     const bool act = v < p;
     const int vc = act ? v : p - 1;
     const float * __restrict__ LU = LU_all + (long long)sysl * RG_ROWS * RG_ROWS;
@@ -5469,12 +5489,18 @@ k_ge_subst_wide(Geom g, const ChunkDesc * __restrict__ chunks, const float * __r
     extern __shared__ __align__(16) float sw_lds[];
     __shared__ int permL[RG_ROWS];
     __shared__ float ring[8][64];   // the newest results
+    __shared__ unsigned char skg[SB_NG];   // skipped steps of each group of eight
     bool sk = false;
+    if (SKIP) __syncthreads();   // the system before is done with the LDS
     if (tid < RG_ROWS) {
         permL[tid] = tid < n ? perm_in[(long long)sysl * g.tc_max + tid] : 0;
         sk = tid < n && skip_in[(long long)sysl * g.tc_max + tid] != 0;
     }
-    if (__syncthreads_or(sk)) return;   // a skipped step: left to k_ge_solve
+    if (SKIP && tid < RG_ROWS) {
+        const unsigned long long m = __ballot(sk);
+        if ((lane & 7) == 0) skg[tid >> 3] = (unsigned char)(m >> lane);
+    }
+    if ((__syncthreads_or(sk) != 0) != SKIP) return;
     // forward
     {
         float (*yl)[64] = reinterpret_cast<float (*)[64]>(sw_lds);
@@ -5492,13 +5518,22 @@ k_ge_subst_wide(Geom g, const ChunkDesc * __restrict__ chunks, const float * __r
             for (int t = 0; t < SB_G; t++) val[q][t] = B[(unsigned)(permL[min(g0 + t, n - 1)] * p + vc)];
         }
         auto finish = [&](int q, int gi) {
-            sb_ftri(val[q], tri[q], std::make_integer_sequence<int, SB_G>{});
+            if constexpr (SKIP)
+                sw_ftri(val[q], tri[q], __builtin_amdgcn_readfirstlane(skg[gi]), std::make_integer_sequence<int, SB_G>{});
+            else
+                sb_ftri(val[q], tri[q], std::make_integer_sequence<int, SB_G>{});
 #pragma unroll
             for (int t = 0; t < SB_G; t++) {
                 const int r = SB_G * gi + t;
                 yl[r][lane] = val[q][t];
                 if (act && r < n) Yt[(unsigned)(r * p + v)] = val[q][t];
             }
+        };
+        auto terms = [&](int q, const float4 & l, const float (&y)[SB_G], int G) {
+            if constexpr (SKIP)
+                sw_fterms(val[q], l, y, __builtin_amdgcn_readfirstlane(skg[G]), std::make_integer_sequence<int, SB_G>{});
+            else
+                sb_fterms(val[q], l, y, std::make_integer_sequence<int, SB_G>{});
         };
         if (wv == 0) finish(0, 0);
         const int ng = (n + SB_G - 1) / SB_G;
@@ -5518,13 +5553,13 @@ k_ge_subst_wide(Geom g, const ChunkDesc * __restrict__ chunks, const float * __r
 #pragma unroll
                 for (int q = 0; q < SW_NQ; q++)
                     if (wv + SW_WAVES * q == G + 1) {
-                        sb_fterms(val[q], lb[k][q], y, std::make_integer_sequence<int, SB_G>{});
+                        terms(q, lb[k][q], y, G);
                         finish(q, G + 1);
                     }
 #pragma unroll
                 for (int q = 0; q < SW_NQ; q++)
                     if (wv + SW_WAVES * q > G + 1 && wv + SW_WAVES * q < ng)
-                        sb_fterms(val[q], lb[k][q], y, std::make_integer_sequence<int, SB_G>{});
+                        terms(q, lb[k][q], y, G);
             }
         }
     }
@@ -5668,6 +5703,53 @@ k_ge_subst_wide(Geom g, const ChunkDesc * __restrict__ chunks, const float * __r
     }
 }
 
+// grid (systems, ceil(p / 64)), 64 * SW_WAVES threads, SW_LDS floats of dynamic LDS
+__global__ void __launch_bounds__(64 * SW_WAVES)
+k_ge_subst_wide(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ aug,
+                const long long * __restrict__ aug_off, const int * __restrict__ perm_in,
+                const unsigned char * __restrict__ skip_in, const float * __restrict__ LU_all, float * Yt_all,
+                float * __restrict__ Cv) {
+    subst_wide<false>(g, chunks, aug, aug_off, perm_in, skip_in, LU_all, Yt_all, Cv, blockIdx.x, blockIdx.y);
+}
+
+// The systems with skipped steps, usually none or a few of many: every block
+// looks through its share of the systems (x, x + gridDim.x, ..) eight at a
+// time, then solves the ones it found. k_ge_solve, which took them one wave
+// per 64 columns before, held a call up for 1.77 ms per such system (256
+// unknowns), 0.3 ms here. grid (blocks, ceil(p / 64)).
+constexpr int SW_LIST = 256;
+
+__global__ void __launch_bounds__(64 * SW_WAVES)
+k_ge_subst_skip(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ aug,
+                const long long * __restrict__ aug_off, const int * __restrict__ perm_in,
+                const unsigned char * __restrict__ skip_in, const float * __restrict__ LU_all, float * Yt_all,
+                float * __restrict__ Cv, int systems) {
+    __shared__ int found[SW_LIST], nfound;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int step = (int)gridDim.x * SW_WAVES;
+    for (int s0 = blockIdx.x; s0 < systems; s0 += step * (SW_LIST / SW_WAVES)) {
+        __syncthreads();
+        if (threadIdx.x == 0) nfound = 0;
+        __syncthreads();
+        for (int k = 0; k < SW_LIST / SW_WAVES; k++) {
+            const int sysl = s0 + k * step + wave * (int)gridDim.x;
+            if (sysl >= systems) break;
+            const int n = chunks[(sysl / g.H) % g.n_chunks].tc;
+            bool sk = false;
+#pragma unroll
+            for (int u = 0; u < RG_ROWS / 64; u++) {
+                const int i = min(lane + 64 * u, n - 1);
+                sk = sk || (n >= 1 && n <= RG_ROWS && skip_in[(long long)sysl * g.tc_max + max(i, 0)] != 0);
+            }
+            if (__ballot(sk) != 0ull && lane == 0) found[atomicAdd(&nfound, 1)] = sysl;
+        }
+        __syncthreads();
+        const int nf = nfound;
+        for (int e = 0; e < nf; e++)
+            subst_wide<true>(g, chunks, aug, aug_off, perm_in, skip_in, LU_all, Yt_all, Cv, found[e], blockIdx.y);
+    }
+}
+
 // general size: physical row swaps in global memory, column-major storage
 __device__ void ge_solve_block(float * __restrict__ a, int n, int p, float * __restrict__ x,
                                long long ldx, float zero_val, float * prow, float * fac) {
@@ -5790,24 +5872,20 @@ __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * _
             int brow = 0x7fffffff;
             for (int r = c + 1 + tid; r < n; r += nt) {
                 const float v = fabsf(Pc[r - c0]);
-                if (v == v && v > best) { best = v; brow = r; }
+                if (v > a0 && __float_as_uint(v) > bk) { bk = __float_as_uint(v); brow = r; }
             }
-            for (int o = 32; o > 0; o >>= 1) {
-                const float ov = __shfl_xor(best, o);
-                const int orow = __shfl_xor(brow, o);
-                if (ov > best || (ov == best && orow < brow)) { best = ov; brow = orow; }
-            }
-            if ((tid & 63) == 0) { bv[tid >> 6] = best; bi[tid >> 6] = brow; }
-            __syncthreads();
-            if (tid == 0) {
-                float b = bv[0];
-                int r = bi[0];
-                for (int i = 1; i < (nt >> 6); i++)
-                    if (bv[i] > b || (bv[i] == b && bi[i] < r)) { b = bv[i]; r = bi[i]; }
-                const float a0 = fabsf(Pc[s]);
-                s_mr[s] = (a0 == a0 && b > a0) ? r : c;
+            {
+                const unsigned km = dpp_reduce_u32<true>(bk);
+                const unsigned rm = dpp_reduce_u32<false>(bk == km ? (unsigned)brow : 0xffffffffu);
+                if ((tid & 63) == 0) { bv[tid >> 6] = km; bi[tid >> 6] = (int)rm; }
             }
             __syncthreads();
+            {
+                const int wl = min(tid & 63, (nt >> 6) - 1);
+                const unsigned kw = bv[wl], km = dpp_reduce_u32<true>(kw);
+                const unsigned rm = dpp_reduce_u32<false>(kw == km ? (unsigned)bi[wl] : 0xffffffffu);
+                s_mr[s] = km != 0u ? (int)rm : c;   // (every thread the same value)
+            }
             const int mr = s_mr[s];
             if (mr != c) {
                 // (the earlier steps' multipliers move with their rows)
@@ -7687,8 +7765,9 @@ constexpr long long SW_MAX_BLOCKS = 256;   // one per CU
 
 void launch_ge_solve(const Geom & g, const Work & w, float * Cv, hipStream_t st) {
     const unsigned systems = (unsigned)(g.L * g.n_chunks * g.H);
-    // k_ge_subst solves every system without a skipped pivot step, k_ge_solve
-    // the others (KVC_SOLVE_OLD=1: k_ge_solve all of them)
+    // k_ge_subst or k_ge_subst_wide solves every system without a skipped pivot
+    // step, k_ge_subst_skip the others (KVC_SOLVE_OLD=1, or without the LDS:
+    // k_ge_solve)
     static const bool old_solve = [] {
         const char * e = getenv("KVC_SOLVE_OLD");
         return e && e[0] == '1';
@@ -7697,6 +7776,9 @@ void launch_ge_solve(const Geom & g, const Work & w, float * Cv, hipStream_t st)
     // every block has its CU, 580 us for 320 of them, where k_ge_subst (eight
     // waves per CU) still takes 420 us
     static const bool wide_ok = hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst_wide),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                    SW_LDS * (int)sizeof(float)) == hipSuccess &&
+                                hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst_skip),
                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
                                                     SW_LDS * (int)sizeof(float)) == hipSuccess;
     if (!old_solve && wide_ok && (long long)systems * cdiv(g.dv, 64) <= SW_MAX_BLOCKS) {
@@ -7713,8 +7795,13 @@ void launch_ge_solve(const Geom & g, const Work & w, float * Cv, hipStream_t st)
         hipLaunchKernelGGL(k_ge_subst, dim3(systems), dim3(64 * nw), lds, st,
                            g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, Cv);
     }
-    hipLaunchKernelGGL(k_ge_solve, dim3(systems, cdiv(g.dv, 64)), dim3(64), 0, st,
-                       g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv, old_solve ? 0 : 1);
+    if (!old_solve && wide_ok)
+        hipLaunchKernelGGL(k_ge_subst_skip, dim3(std::min(systems, 256u), cdiv(g.dv, 64)), dim3(64 * SW_WAVES),
+                           SW_LDS * sizeof(float), st, g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv,
+                           (int)systems);
+    else
+        hipLaunchKernelGGL(k_ge_solve, dim3(systems, cdiv(g.dv, 64)), dim3(64), 0, st,
+                           g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv, old_solve ? 0 : 1);
     if (g.tc_max > RG_ROWS) {
         // dynamic LDS: the largest system's panels (3 pb n floats), or the
         // step-by-step factors; the attribute once per process

@@ -103,3 +103,22 @@ def test_substitution_wide_edges(gpu, orc, n, d):
     b = orc.compact(K, V, Q, T, nq, 2, d, d, orc.params(target_ratio=0.5, chunk_size=-1))
     assert a.t == b.t == n and np.array_equal(a.indices, b.indices)
     assert np.array_equal(a.C_v.view(np.uint32), b.C_v.view(np.uint32)), "C_v"
+
+
+# Systems with skipped pivots: equal keys make M exactly singular, and the beta
+# fit's ridge of 1e-10 is lost beside its entries. One system (all of the
+# grid), several chunks, and column counts past one block of 64.
+@pytest.mark.parametrize("T,H,d,nq,chunk,ratio", [
+    (6, 1, 32, 4, -1, 0.5), (40, 2, 64, 9, -1, 0.5), (130, 1, 130, 40, -1, 0.5), (256, 2, 64, 24, -1, 0.5),
+    (400, 1, 128, 64, -1, 0.5), (512, 2, 96, 32, -1, 0.5), (3000, 2, 64, 32, 300, 0.4)])
+def test_skipped_pivots(gpu, orc, T, H, d, nq, chunk, ratio):
+    K, V = kv_cache(T, H, d, 71)
+    K[1::2] = K[0::2][:T // 2]
+    Q = snapkv_queries(K, nq, 71)
+    print(f"[skip] T={T} H={H} d={d} nq={nq} chunk={chunk}", flush=True)
+    par = dict(target_ratio=ratio, chunk_size=chunk, skip_beta=0, nnls_method=1)
+    a = gpu.compact(K, V, Q, T, nq, H, d, d, gpu.params(**par))
+    b = orc.compact(K, V, Q, T, nq, H, d, d, orc.params(**par))
+    assert a.t == b.t and np.array_equal(a.indices, b.indices)
+    assert np.array_equal(a.beta.view(np.uint32), b.beta.view(np.uint32)), "beta"
+    assert np.array_equal(a.C_v.view(np.uint32), b.C_v.view(np.uint32)), "C_v"

@@ -314,3 +314,19 @@ def test_refit_target_blocks(gpu, orc, T, H, d, nq, chunk):
     assert np.array_equal(a.C_v.view(np.uint32), b.C_v.view(np.uint32)), "C_v"
     for k in ("avg_cosine_sim", "avg_mse", "avg_agreement"):
         assert np.float32(a.stats[k]).view(np.uint32) == np.float32(b.stats[k]).view(np.uint32), k
+
+
+# Keys in equal pairs with an odd kept count: the pair at the boundary ties,
+# and the heap selection decides which of the two stays. Sizes on both sides
+# of its LDS forms.
+@pytest.mark.parametrize("T,t", [(2, 1), (10, 3), (130, 65), (300, 129), (2048, 255), (4600, 101), (4800, 101), (7200, 37)])
+def test_boundary_ties(gpu, orc, T, t):
+    print(f"[ties] T={T} t={t}", flush=True)
+    K, V = kv_cache(T, 1, 32, 67)
+    K[1::2] = K[0::2][:T // 2]
+    Q = snapkv_queries(K, min(T, 8), 67)
+    par = dict(target_count=t, chunk_size=-1)
+    a = gpu.compact(K, V, Q, T, len(Q), 1, 32, 32, gpu.params(**par))
+    b = orc.compact(K, V, Q, T, len(Q), 1, 32, 32, orc.params(**par))
+    assert a.t == t
+    same(a, b)
