@@ -5837,7 +5837,7 @@ constexpr int GE_LDS_FLOATS = 8192;
 //     per thread, then a[r][j] -= F[s][r] * U12[s][j], s ascending, for the
 //     rows below in register tiles (below). Each column in LDS by 16 lanes,
 //     two LDS reads and a write per term, took the 256 systems of 409 + 128
-//     columns 8.8 ms; 5.6 ms in tiles, of which most is now the panels' serial
+//     columns 8.8 ms; 4.3 ms now, of which most is now the panels' serial
 //     steps and the back substitution's chain.
 // Then the back substitution of ge_solve_block. Dynamic LDS: 3 pb nr floats
 // (F, P and the row map, then F, U12 and the row map; nr rounded up to 4).
@@ -6023,6 +6023,106 @@ __device__ void ge_solve_blocked(float * __restrict__ a, int n, int p, float * _
         }
         __syncthreads();
     }
+    // Back substitution (the order of ge_solve_block's), a column per lane and
+    // 64 columns per wave: y, then x in place, in LDS as blocks of four rows
+    // ({row 4 b .. 4 b + 3} of a lane at X[(64 b + lane) 4]), U row col
+    // (contiguous at a[col n + col ..]) in one of two LDS rows, the next one
+    // loaded by the whole block meanwhile. Four terms are two 16-byte reads,
+    // the next sixteen's under way while sixteen are subtracted; entries past n
+    // are 0 (v - 0 = v). 409 unknowns, 128 columns: 2.9 -> 1.9 ms of the 256
+    // systems' time against one row and one entry per read.
+    {
+        const int n4 = (n + 3) & ~3, nb = n4 >> 2, us = n4 + 16, xs = (nb + 4) * 256;
+        const int waves = min((3 * pb * n4 - 2 * us) / xs, nt >> 6);
+        if (waves >= 1) {
+            float * ub = lds, * X = lds + 2 * us;
+            const int wv = tid >> 6, lane = tid & 63;
+            float * Xw = X + wv * xs + 4 * lane;
+            constexpr int PF = 4;
+            for (int j0 = 0; j0 < p; j0 += 64 * waves) {
+                const int nc = min(64 * waves, p - j0), wn = (nc + 63) >> 6;
+                __syncthreads();
+                for (int e = tid; e < wn * xs; e += nt) X[e] = 0.0f;
+                for (int e = n + tid; e < us; e += nt) ub[e] = ub[us + e] = 0.0f;
+                if (tid == 0) ub[((n - 1) & 1) * us + n - 1] = a[(long long)(n - 1) * n + n - 1];
+                __syncthreads();
+                for (int e = tid; e < nc * n; e += nt) {
+                    const int j = e / n, r = e - j * n;
+                    X[(j >> 6) * xs + (r >> 2) * 256 + 4 * (j & 63) + (r & 3)] = a[(long long)(n + j0 + j) * n + r];
+                }
+                __syncthreads();
+                for (int col = n - 1; col >= 0; col--) {
+                    // row col - 1 (entries col - 1 .. n - 1) toward the other buffer
+                    const int nld = col > 0 ? n - col + 1 : 0;
+                    const float * src = a + (long long)(col - 1) * n + (col - 1);
+                    float * dst = ub + ((col - 1) & 1) * us + (col - 1);
+                    float pre[PF];
+#pragma unroll
+                    for (int k = 0; k < PF; k++) pre[k] = tid + k * nt < nld ? src[tid + k * nt] : 0.0f;
+                    if (wv < wn) {
+                        const float * u = ub + (col & 1) * us;
+                        const float piv = u[col];
+                        float v = zero_val;
+                        if (!(fabsf(piv) < 1e-12f)) {
+                            v = Xw[(col >> 2) * 256 + (col & 3)];
+                            int b = (col + 1) >> 2;
+                            if ((col + 1) & 3) {   // the rest of row col's block
+                                const float4 uv = *reinterpret_cast<const float4 *>(&u[4 * b]);
+                                const float4 xv = *reinterpret_cast<const float4 *>(&Xw[b * 256]);
+                                if (4 * b + 1 > col) v = v - uv.y * xv.y;
+                                if (4 * b + 2 > col) v = v - uv.z * xv.z;
+                                v = v - uv.w * xv.w;
+                                b++;
+                            }
+                            float4 uq[2][4], xq[2][4];
+                            auto get = [&](int s, int at) {   // (blocks nb .. nb + 3 are zeros)
+                                at = min(at, nb);
+#pragma unroll
+                                for (int m = 0; m < 4; m++) {
+                                    uq[s][m] = *reinterpret_cast<const float4 *>(&u[4 * (at + m)]);
+                                    xq[s][m] = *reinterpret_cast<const float4 *>(&Xw[(at + m) * 256]);
+                                }
+                                asm volatile("" ::: "memory");   // keeps the loads ahead of the sums
+                            };
+                            auto take = [&](int s) {
+#pragma unroll
+                                for (int m = 0; m < 4; m++) {
+                                    v = v - uq[s][m].x * xq[s][m].x;
+                                    v = v - uq[s][m].y * xq[s][m].y;
+                                    v = v - uq[s][m].z * xq[s][m].z;
+                                    v = v - uq[s][m].w * xq[s][m].w;
+                                }
+                                asm volatile("" : "+v"(v));
+                            };
+                            if (b < nb) {
+                                get(0, b);
+                                for (;; b += 8) {
+                                    get(1, b + 4);
+                                    take(0);
+                                    if (b + 4 >= nb) break;
+                                    get(0, b + 8);
+                                    take(1);
+                                    if (b + 8 >= nb) break;
+                                }
+                            }
+                            v = v / piv;
+                        }
+                        Xw[(col >> 2) * 256 + (col & 3)] = v;
+                    }
+#pragma unroll
+                    for (int k = 0; k < PF; k++)
+                        if (tid + k * nt < nld) dst[tid + k * nt] = pre[k];
+                    __syncthreads();
+                }
+                for (int e = tid; e < n * nc; e += nt) {
+                    const int r = e / nc, j = e - r * nc;
+                    x[(long long)r * ldx + j0 + j] = X[(j >> 6) * xs + (r >> 2) * 256 + 4 * (j & 63) + (r & 3)];
+                }
+            }
+            return;
+        }
+    }
+    // larger systems:
     // back substitution (the order of ge_solve_block's) from LDS, in passes
     // of pc right-hand-side columns: the pass's y, then x in place, at
     // xl[r (pc + 1) + j]; U row col (contiguous at a[col n + col ..]) in one
