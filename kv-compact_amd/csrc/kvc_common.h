@@ -43,6 +43,12 @@ struct RowCodec {
     int type;               // KV_TYPE_Q8_0 (8) or KV_TYPE_Q4_0 (2)
 };
 
+// A state blob's K or V section header (12 bytes used) and its byte offset.
+struct HeaderBytes {
+    unsigned long long at;
+    uint8_t b[16];
+};
+
 // Geometry of a batch of layers sharing one plan.
 struct Geom {
     int L, T, H, dk, dv;

@@ -2391,6 +2391,7 @@ StateRun state_compact_impl(const uint8_t * blob, size_t size, bool dev, const k
         float * zbeta = nullptr, * beta_c = nullptr, * Cv = nullptr, * stats = nullptr, * dirs = nullptr;
         float * rows = nullptr, * cols = nullptr;
         uint8_t * stage = nullptr;
+        HeaderBytes * hdrs = nullptr;
         Work w{}, wd{};
     };
     auto carve = [&](Carver & c, Bufs & b) {
@@ -2407,6 +2408,7 @@ StateRun state_compact_impl(const uint8_t * blob, size_t size, bool dev, const k
         b.dirs = c.take<float>((size_t)L * H * dk);
         b.rows = c.take<float>((size_t)t * std::max(nk, nv));
         b.cols = c.take<float>((size_t)nv * t);
+        b.hdrs = c.take<HeaderBytes>((size_t)2 * L);
         b.stage = c.take<uint8_t>(size);   // the compacted blob is never larger than the input
         if (Lc > 0) {
             StatWork sw{};
@@ -2504,9 +2506,7 @@ StateRun state_compact_impl(const uint8_t * blob, size_t size, bool dev, const k
         gg.H = Lc * H;
         launch_global_importance(gg, w, st);
         launch_select_topk(gg, w, st);
-        for (int l = 1; l < Lc; l++)
-            if (hipMemcpyAsync(idx + (size_t)l * t, idx, (size_t)t * 4, hipMemcpyDeviceToDevice, st) != hipSuccess)
-                return done(KV_COMPACT_E_DEVICE);
+        launch_repeat_int(idx, t, Lc - 1, st);
         launch_refit_target(g, w, io.V, st);
         launch_fill_f32(b.beta_c, 0.0f, (long long)Lc * H * t, st);
         launch_ls_softmax(g, w, b.beta_c, st);
@@ -2578,16 +2578,30 @@ StateRun state_compact_impl(const uint8_t * blob, size_t size, bool dev, const k
     }
     if (hipMemcpyAsync(stage, hdr.data(), hdr.size(), hipMemcpyHostToDevice, st) != hipSuccess)
         return done(KV_COMPACT_E_DEVICE);
-    std::vector<uint8_t> lh((size_t)2 * L * 16);
+    std::vector<HeaderBytes> lh((size_t)2 * L);   // K headers, then V headers
+    for (int l = 0; l < L; l++) {
+        const StateLayer & ld = s.layers[l];
+        HeaderBytes & kh = lh[l], & vh = lh[(size_t)L + l];
+        kh.at = o.k_hdr[l];
+        memcpy(kh.b, &ld.k_type, 4);
+        memcpy(kh.b + 4, &ld.k_rb, 8);
+        vh.at = o.v_hdr[l];
+        memcpy(vh.b, &ld.v_type, 4);
+        if (!s.v_trans) {
+            memcpy(vh.b + 4, &ld.v_rb, 8);
+        } else {
+            const uint32_t ne = (uint32_t)(H * dv);
+            memcpy(vh.b + 4, &ld.v_el, 4);
+            memcpy(vh.b + 8, &ne, 4);
+        }
+    }
+    if (hipMemcpyAsync(b.hdrs, lh.data(), lh.size() * sizeof(HeaderBytes), hipMemcpyHostToDevice, st) != hipSuccess)
+        return done(KV_COMPACT_E_DEVICE);
+    launch_put_headers(b.hdrs, 2 * L, stage, st);
     (void)hipEventRecord(ctx->q_ev[2], st);
     const float scale = sqrtf((float)dk);
     for (int l = 0; l < L; l++) {
         const StateLayer & ld = s.layers[l];
-        uint8_t * kh = lh.data() + (size_t)l * 16;
-        memcpy(kh, &ld.k_type, 4);
-        memcpy(kh + 4, &ld.k_rb, 8);
-        if (hipMemcpyAsync(stage + o.k_hdr[l], kh, 12, hipMemcpyHostToDevice, st) != hipSuccess)
-            return done(KV_COMPACT_E_DEVICE);
         const int sl = slot[l];
         const int * sidx = idx;   // row 0: every layer keeps the same cells
         launch_fold_rows(Kf + (size_t)sl * T * nk, nk, sidx, t, zbeta, dirs + (size_t)sl * H * dk, H, dk, scale,
@@ -2597,14 +2611,11 @@ StateRun state_compact_impl(const uint8_t * blob, size_t size, bool dev, const k
     }
     for (int l = 0; l < L; l++) {
         const StateLayer & ld = s.layers[l];
-        uint8_t * vh = lh.data() + (size_t)(L + l) * 16;
-        memcpy(vh, &ld.v_type, 4);
         const int sl = slot[l];
         const bool comp = sl < Lc;
         const float * cvl = comp ? Cv + (size_t)sl * H * t * dv : nullptr;
         const float * vl = Vf + (size_t)sl * T * nv;
         if (!s.v_trans) {
-            memcpy(vh + 4, &ld.v_rb, 8);
             if (comp) {
                 launch_gather_cv_rows(cvl, H, t, dv, rows, st);
                 encode_rows(rows, nv, nullptr, iota, ld.v_type, nv, t, stage + o.v_pay[l], o.v_w[l], st);
@@ -2613,14 +2624,10 @@ StateRun state_compact_impl(const uint8_t * blob, size_t size, bool dev, const k
             }
         } else {
             const uint32_t ne = (uint32_t)(H * dv);
-            memcpy(vh + 4, &ld.v_el, 4);
-            memcpy(vh + 8, &ne, 4);
             launch_value_columns(cvl, vl, nv, idx, H, dv, t, cols, st);
             launch_quant_rows(cols, t, nullptr, ld.v_type, t, (long long)ne, stage + o.v_pay[l],
                               (long long)o.v_w[l], st);
         }
-        if (hipMemcpyAsync(stage + o.v_hdr[l], vh, 12, hipMemcpyHostToDevice, st) != hipSuccess)
-            return done(KV_COMPACT_E_DEVICE);
     }
     (void)hipEventRecord(ctx->q_ev[3], st);
     // empty streams and the trailing bytes

@@ -89,6 +89,8 @@ void launch_value_columns(const float * Cv, const float * V, int nv, const int *
                           float * col, hipStream_t st);
 void launch_gather_qref(const float * K, long long ldK, int nk, int q0, int nq, int H, int dk, int L, float * out,
                         hipStream_t st);
+void launch_repeat_int(int * p, int n, int times, hipStream_t st);
+void launch_put_headers(const HeaderBytes * h, int n, uint8_t * dst, hipStream_t st);
 void launch_iota(int * p, long long n, hipStream_t st);
 void launch_gemm_abt(const float * A, long long lda, const float * B, long long ldb, float * C, long long ldc,
                      int m, int n, int k, float scale, long long sa, long long sb, long long sc, int batch,

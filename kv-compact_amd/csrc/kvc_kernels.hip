@@ -7524,6 +7524,22 @@ k_gather_qref(const float * __restrict__ K, long long ldK, int nk, int q0, int n
     }
 }
 
+// p[0 .. n - 1] again at p + n, p + 2 n, .. (grid y)
+__global__ void __launch_bounds__(256) k_repeat_int(int * __restrict__ p, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[(long long)(blockIdx.y + 1) * n + i] = p[i];
+}
+
+// the twelve-byte headers of a blob's layers to their places (any alignment):
+// one upload and one launch for all of them
+__global__ void __launch_bounds__(64) k_put_headers(const HeaderBytes * __restrict__ h, int n, uint8_t * __restrict__ dst) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i >= n) return;
+    const HeaderBytes x = h[i];
+#pragma unroll
+    for (int k = 0; k < 12; k++) dst[x.at + k] = x.b[k];
+}
+
 __global__ void __launch_bounds__(256) k_iota(int * __restrict__ p, long long n) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = (int)i;
@@ -8157,6 +8173,15 @@ void launch_gather_qref(const float * K, long long ldK, int nk, int q0, int nq, 
     if (L <= 0) return;
     hipLaunchKernelGGL(k_gather_qref, dim3(grid_cap((long long)H * nq * dk, 256), L), dim3(256), 0, st,
                        K, ldK, nk, q0, nq, H, dk, out);
+}
+
+void launch_repeat_int(int * p, int n, int times, hipStream_t st) {
+    if (n > 0 && times > 0)
+        hipLaunchKernelGGL(k_repeat_int, dim3(cdiv(n, 256), times), dim3(256), 0, st, p, n);
+}
+
+void launch_put_headers(const HeaderBytes * h, int n, uint8_t * dst, hipStream_t st) {
+    if (n > 0) hipLaunchKernelGGL(k_put_headers, dim3(cdiv(n, 64)), dim3(64), 0, st, h, n, dst);
 }
 
 void launch_iota(int * p, long long n, hipStream_t st) {
