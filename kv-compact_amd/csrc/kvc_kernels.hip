@@ -1021,13 +1021,14 @@ k_refit_target(Geom g, const ChunkDesc * __restrict__ chunks, const float * __re
     const int c_idx = blockIdx.x / g.H, h = blockIdx.x % g.H, layer = blockIdx.y;
     const ChunkDesc c = chunks[c_idx];
     const long long ev = (long long)g.H * g.dv;
-    const int nv = g.dv / VB, v0 = ((int)blockIdx.z % nv) * VB, q0 = ((int)blockIdx.z / nv) * QB;
-    if (q0 >= c.nq || c.Tc <= 0) return;
+    const int nv = g.dv / VB, v0 = ((int)blockIdx.z % nv) * VB, nzq = (int)gridDim.z / nv;
+    if (c.Tc <= 0) return;
     const long long sys = ((long long)layer * g.n_chunks + c_idx) * g.H + h;
-    attn_sum_block<VC, VB, QB>(A + layer * lS(g) + h * hS(g) + c.start, ainv + sys * g.nq_max, g.T, q0, c.nq,
-                 VC ? nullptr : V + layer * g.ldV + (long long)c.start * ev + (long long)h * g.dv + v0, ev, c.Tc,
-                 Y + sys * g.nq_max * g.dv + v0, g.dv,
-                 g.vc, layer, c.start, h * g.dv + v0);
+    for (int q0 = ((int)blockIdx.z / nv) * QB; q0 < c.nq; q0 += nzq * QB)
+        attn_sum_block<VC, VB, QB>(A + layer * lS(g) + h * hS(g) + c.start, ainv + sys * g.nq_max, g.T, q0, c.nq,
+                     VC ? nullptr : V + layer * g.ldV + (long long)c.start * ev + (long long)h * g.dv + v0, ev, c.Tc,
+                     Y + sys * g.nq_max * g.dv + v0, g.dv,
+                     g.vc, layer, c.start, h * g.dv + v0);
 }
 
 template <int VC>
@@ -3431,7 +3432,8 @@ k_ls_build(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restri
 // that step on, r's U row; plus the final permutation and the skipped-pivot
 // flags. The right-hand sides are not touched here: the reference's
 // elimination of them is forward substitution with the final permutation
-// (ascending steps), done with the back substitution in k_ge_solve.
+// (ascending steps), done with the back substitution in k_ge_subst and its
+// relatives.
 // ---------------------------------------------------------------------------
 constexpr int RG_ROWS = 256, RG_WAVES = 16, RG_COLS = 16, RG_SLOTS = 4;
 constexpr int RG_THREADS = RG_WAVES * 64;
@@ -5337,7 +5339,7 @@ k_ge_subst(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restri
     extern __shared__ float sb_lds[];
     float (*zl)[64] = reinterpret_cast<float (*)[64]>(sb_lds + (size_t)wv * SB_LROWS * 64);
     // permutation by logical row (lane l holds rows l, l + 64, ...); a system
-    // with a skipped step is left to k_ge_solve
+    // with a skipped step is left to k_ge_subst_skip
     int pv[4];
     bool sk = false;
 #pragma unroll
@@ -6722,7 +6724,7 @@ k_stats_final(Geom g, const float * __restrict__ oo, const float * __restrict__ 
     const float * c = co + (long long)layer * nt * g.dv;
     // thread i owns output row i; the rows pass through LDS in slabs of
     // columns, so that memory is read along them (one row per thread straight
-    // from memory took 70 us for 128 rows of 128, this 9)
+    // from memory took 70 us for 128 rows of 128, this 9, 18 for 32 layers)
     float dp = 0.0f, no = 0.0f, nc = 0.0f, mse = 0.0f, mo = 0.0f, mc = 0.0f;
     int ao = 0, ac = 0;
     for (int d0 = 0; d0 < g.dv; d0 += SF_DT) {
@@ -7638,12 +7640,13 @@ void launch_chunk_softmax(const Geom & g, const Work & w, hipStream_t st) {
 }
 
 constexpr long long RT_NARROW = 320, RT_WIDE = 1024;
+constexpr unsigned RT_SPARE_LDS = 11 * 1024;
 
 template <int VC>
 void launch_refit_inst(const Geom & g, const Work & w, const float * V, bool aligned, hipStream_t st) {
     const dim3 grid(g.n_chunks * g.H, g.L);
-    auto go = [&](auto kernel, unsigned z) {
-        hipLaunchKernelGGL(kernel, dim3(grid.x, grid.y, z), dim3(256), 0, st, g, w.chunks, w.A, w.ainv, V, w.Y);
+    auto go = [&](auto kernel, unsigned z, unsigned lds = 0) {
+        hipLaunchKernelGGL(kernel, dim3(grid.x, grid.y, z), dim3(256), lds, st, g, w.chunks, w.A, w.ainv, V, w.Y);
     };
     // Column blocks as wide as d_v allows. Queries 64 at a time (a 64- or
     // 32-column block then gives a thread 4 or 2 x 4 sums) where that still
@@ -7658,7 +7661,14 @@ void launch_refit_inst(const Geom & g, const Work & w, const float * V, bool ali
     } else if (!aligned || vb == 0) {
         go(k_refit_target_any<VC>, q32);
     } else if (vb == 128) {
-        go(k_refit_target<VC, 128, 32>, q32 * (g.dv / 128));
+        // five blocks per CU (the unused LDS; its registers would allow seven):
+        // with more, the diversity Gram beside it gets less of the chip than
+        // it needs to finish with it (100k tokens, 32 layers: the Gram 8.8 ms
+        // at five, 10.4 at seven, the refit target 11.4 and 10.1)
+        // (a unit's query blocks in one block, its values still in L2, where the
+        // units alone fill the chip)
+        const unsigned nv = g.dv / 128;
+        go(k_refit_target<VC, 128, 32>, (units * nv >= 2048 ? 1 : q32) * nv, RT_SPARE_LDS);
     } else {
         const unsigned nv = g.dv / vb;
         const bool wide = g.nq_max > 32 && units * q64 * nv >= RT_WIDE;
