@@ -2693,7 +2693,12 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
 
 // Two waves' offer for a step: each wave's best pivot row, from the block's
 // first column on (two sets, by the step's parity: a slower wave may still be
-// reading the step before).
+// reading the step before). The barrier between a step's writes and its reads
+// also orders the step before: its U row and ub are written, and its offers
+// read, by then. The last step of an elimination has no later one, so the
+// block meets once more before the back substitution; without that a wave
+// could read the U row of the sub-problem before, or write the next one's
+// first offer over one that the other still reads.
 template <int W>
 struct LhOffer {
     unsigned key, first;   // |pivot|, and the first position that has it
@@ -2961,7 +2966,8 @@ k_nnls_lh(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restric
                         for (int k = k0; k < k0 + 16 && k + LH_SB < K; k++) a[k] = a[k + LH_SB];
                     }
             }
-            wave_sync();
+            if constexpr (W == 2) __syncthreads();   // the last step's U row and ub, and its offers read (LhOffer)
+            else wave_sync();
             // back substitution: x[q] is the value of passive index lane + 64 q;
             // the next column's entries load while one is summed
             float x[W], un[W], pvn = 0.0f, bn = 0.0f;
