@@ -2701,10 +2701,11 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
 // first offer over one that the other still reads.
 template <int W>
 struct LhOffer {
-    unsigned key, first;   // |pivot|, and the first position that has it
+    alignas(16) float row[64 * W];   // (written four at a time)
+    unsigned key, first;             // |pivot|, and the first position that has it
     float b;
-    float row[64 * W];
 };
+static_assert(sizeof(LhOffer<2>) % 16 == 0, "every offer's row is aligned");
 
 // Step c0 + J of the elimination: pivot, the pivot row's entries from column
 // c0 on to U (at base, which moves past them) and ub, and the update of the
@@ -2848,7 +2849,7 @@ k_nnls_lh(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restric
     __shared__ __align__(16) float U[UF];
     __shared__ float ub[K], svs[W][256], lws[W][K];
     __shared__ int ljs[W][K];
-    __shared__ __align__(16) LhOffer<W> offer[W][W];   // (used by two waves)
+    __shared__ LhOffer<W> offer[W][W];   // (used by two waves)
     float * sv = svs[wave], * lw = lws[wave];   // (one copy per wave: a wave may be ahead)
     int * lj = ljs[wave];
     float w[4], grad[4], atb[4], pw[4], p2w[4], bw[4];   // w, and the states it is compared with

@@ -1,6 +1,6 @@
 """k_nnls_lh lane by lane on the CPU (tests/waves): what passes between the
-two waves of a block is ordered by block barriers whichever wave runs first.
-Every case's weights equal the oracle's bit for bit."""
+two waves of a block is ordered by block barriers whichever wave runs first,
+and no LDS access is misaligned. Every case's weights equal the oracle's bit for bit."""
 from __future__ import annotations
 
 import ctypes
@@ -30,8 +30,8 @@ def model(tmp_path_factory):
     # (the one register constraint by the host's name)
     (d / "lawson_hanson.inc").write_text(m.group(0).replace('"+v"(me)', '"+r"(me)'))
     exe = d / "lawson_hanson"
-    b = subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-w", "-ffp-contract=off",
-                        f"-I{d}", str(HERE / "waves" / "lawson_hanson.cpp"),
+    b = subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-w", "-ffp-contract=off", "-fsanitize=undefined",
+                        "-fno-sanitize-recover=undefined", f"-I{d}", str(HERE / "waves" / "lawson_hanson.cpp"),
                         "-o", str(exe)], capture_output=True, text=True, timeout=300)
     assert b.returncode == 0, b.stderr[-3000:]
     return exe
