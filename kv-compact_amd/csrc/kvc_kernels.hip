@@ -2982,7 +2982,7 @@ k_nnls_lh(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restric
                 pvn = U[base + col - c0];
                 bn = ub[col];
             };
-            fetch(pc - 1);
+            if (pc > 0) fetch(pc - 1);   // (a boundary step may have emptied the set: s is 0 then)
             for (int col = pc - 1; col >= 0; col--) {
                 float prod[W], val = bn;
                 const float piv = pvn;

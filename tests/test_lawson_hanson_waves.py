@@ -1,6 +1,7 @@
 """k_nnls_lh lane by lane on the CPU (tests/waves): what passes between the
 two waves of a block is ordered by block barriers whichever wave runs first,
-and no LDS access is misaligned. Every case's weights equal the oracle's bit for bit."""
+and no LDS access is misaligned or out of range. Every case's weights equal
+the oracle's bit for bit."""
 from __future__ import annotations
 
 import ctypes
@@ -67,14 +68,18 @@ def system(m, n, seed, form=""):
         M = (M * 0.02 + 3.0 * np.eye(m, n)).astype(np.float32)
     if form == "repeat":   # ties, and sub-problems that are singular but for the 1e-10
         M[:, 1::2] = M[:, 0::2][:, :n // 2]
+    if form == "huge":     # a column whose own weight comes out 0: the set empties at once
+        M[:, n // 2] = np.float32(1e20)
     b = (M.sum(1) * ((1.5 if form == "apart" else 0.5) + uniform(seed + 1, m))).astype(np.float32)
+    if form == "huge":
+        b = np.ones(m, np.float32)
     return np.ascontiguousarray(M), b
 
 
 # Passive sets of odd and even size (the step's parity picks the offer), one
 # variable, sets past 64 (both waves have rows), caps that end a loop early.
 CASES = [(6, 1, 3, 200, ""), (4, 3, 5, 200, ""), (9, 7, 11, 200, ""), (16, 13, 13, 60, ""), (12, 24, 17, 40, ""),
-         (8, 12, 19, 40, "repeat"), (72, 71, 31, 200, "apart")]
+         (8, 12, 19, 40, "repeat"), (3, 5, 23, 7, "huge"), (72, 71, 31, 200, "apart")]
 
 
 @pytest.mark.parametrize("first", [0, 1])

@@ -4,7 +4,8 @@
 // only. Between two block barriers the scheduler runs one wave as far as it
 // goes before the other starts, in the order the test names, so a value that
 // passes between the waves without a barrier is read stale or overwritten
-// every time. LDS arrays are statics, (see the test for what is compared).
+// every time. LDS arrays are statics, which the undefined-behaviour
+// sanitizer bounds and aligns.
 //
 // stdin: int32 waves, first wave to run, n, max_iter; n (n + 1) floats
 // [AtA | Atb]. stdout: n floats; the status word and the redo flag as int32.
