@@ -7896,6 +7896,12 @@ void launch_ge_lu(const Geom & g, const Work & w, hipStream_t st, bool m_by_lu) 
 
 constexpr long long SW_MAX_BLOCKS = 256;   // one per CU
 
+// KVC_SUBST_WIDE=0 (read at every launch) solves small grids by k_ge_subst too
+static bool subst_wide_enabled() {
+    const char * e = getenv("KVC_SUBST_WIDE");
+    return !(e && e[0] == '0');
+}
+
 void launch_ge_solve(const Geom & g, const Work & w, float * Cv, hipStream_t st) {
     const unsigned systems = (unsigned)(g.L * g.n_chunks * g.H);
     // k_ge_subst or k_ge_subst_wide solves every system without a skipped pivot
@@ -7914,7 +7920,7 @@ void launch_ge_solve(const Geom & g, const Work & w, float * Cv, hipStream_t st)
                                 hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst_skip),
                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
                                                     SW_LDS * (int)sizeof(float)) == hipSuccess;
-    if (!old_solve && wide_ok && (long long)systems * cdiv(g.dv, 64) <= SW_MAX_BLOCKS) {
+    if (!old_solve && wide_ok && subst_wide_enabled() && (long long)systems * cdiv(g.dv, 64) <= SW_MAX_BLOCKS) {
         hipLaunchKernelGGL(k_ge_subst_wide, dim3(systems, cdiv(g.dv, 64)), dim3(64 * SW_WAVES),
                            SW_LDS * sizeof(float), st, g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv);
     } else if (!old_solve) {

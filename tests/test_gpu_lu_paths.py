@@ -90,10 +90,23 @@ def test_nonfinite_inputs(gpu, orc, name, pgd):
 # The substitution that spreads a system over eight waves (grids of at most
 # one block per CU): unknown counts around its groups of eight rows and blocks
 # of four entries, column counts around its 64 lanes.
-@pytest.mark.parametrize("n,d", [(1, 32), (2, 40), (3, 64), (4, 72), (5, 130), (8, 32), (9, 64), (31, 96), (33, 64),
-                                 (64, 256), (127, 40), (129, 64), (201, 72), (253, 64), (254, 130), (255, 64),
-                                 (256, 128)])
+SUBST_EDGES = [(1, 32), (2, 40), (3, 64), (4, 72), (5, 130), (8, 32), (9, 64), (31, 96), (33, 64), (64, 256), (127, 40),
+               (129, 64), (201, 72), (253, 64), (254, 130), (255, 64), (256, 128)]
+
+
+@pytest.mark.parametrize("n,d", SUBST_EDGES)
 def test_substitution_wide_edges(gpu, orc, n, d):
+    check_substitution(gpu, orc, n, d)
+
+
+# The same with the one wave per 64 columns that larger grids take.
+@pytest.mark.parametrize("n,d", SUBST_EDGES)
+def test_substitution_one_wave_edges(gpu, orc, n, d, monkeypatch):
+    monkeypatch.setenv("KVC_SUBST_WIDE", "0")
+    check_substitution(gpu, orc, n, d)
+
+
+def check_substitution(gpu, orc, n, d):
     T = 2 * n
     K, V = kv_cache(T, 2, d, 61, channel_scale=True)
     nq = min(T, 24)
