@@ -135,3 +135,30 @@ def test_skipped_pivots(gpu, orc, T, H, d, nq, chunk, ratio):
     assert a.t == b.t and np.array_equal(a.indices, b.indices)
     assert np.array_equal(a.beta.view(np.uint32), b.beta.view(np.uint32)), "beta"
     assert np.array_equal(a.C_v.view(np.uint32), b.C_v.view(np.uint32)), "C_v"
+
+
+# Skipped pivots in the value refit, many columns a system: without its ridge a
+# pair of equal keys gives a pivot that cancels exactly. At most 256 unknowns
+# (columns past one block of 64), then the blocked elimination: full panels,
+# narrower ones with sizes that are no multiple of four, and the sizes whose
+# back substitution does not fit LDS 64 columns at a time; with and without
+# skipped pivots, and the beta fit's single column beside them.
+@pytest.mark.parametrize("T,H,d,nq,pairs", [
+    (6, 1, 130, 4, 1), (130, 1, 130, 40, 1), (512, 2, 96, 32, 1), (514, 1, 40, 40, 1), (700, 2, 40, 64, 1),
+    (1042, 1, 130, 400, 1), (1042, 1, 130, 24, 1), (1160, 1, 64, 33, 1), (1202, 1, 72, 64, 1), (1042, 1, 130, 400, 0),
+    (1178, 1, 64, 200, 0)])
+def test_skipped_pivots_values(gpu, orc, T, H, d, nq, pairs):
+    K, V = kv_cache(T, H, d, 71)
+    if pairs:
+        K[1::2] = K[0::2][:T // 2]
+    Q = snapkv_queries(K, nq, 71)
+    print(f"[skip] values T={T} H={H} d={d} nq={nq} pairs={pairs}", flush=True)
+    for par in (dict(skip_beta=1, ridge=0.0 if pairs else 1e-6), dict(skip_beta=0, nnls_method=1)):
+        par.update(target_ratio=0.5, chunk_size=-1)
+        a = gpu.compact(K, V, Q, T, nq, H, d, d, gpu.params(**par))
+        b = orc.compact(K, V, Q, T, nq, H, d, d, orc.params(**par))
+        # a skipped pivot's values are exactly 0
+        assert not par["skip_beta"] or (b.C_v == 0).all(-1).any() == bool(pairs)
+        assert a.t == b.t == T // 2 and np.array_equal(a.indices, b.indices)
+        assert np.array_equal(a.beta.view(np.uint32), b.beta.view(np.uint32)), "beta"
+        assert np.array_equal(a.C_v.view(np.uint32), b.C_v.view(np.uint32)), "C_v"
