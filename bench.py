@@ -52,7 +52,7 @@ QSTAGES = STAGES + ["dequantize", "requantize"]
 STAGE_KERNELS = {"scores": "k_scores", "chunk_softmax_importance": "k_softmax_importance",
                  "refit_target": "k_refit_target",
                  "selection": "k_global_importance + k_select_topk (or k_div_candidates + k_div_gram + k_div_greedy)",
-                 "beta_fit": "k_gather_exp + k_ls_build + k_ge_lu + k_ge_solve (or k_nnls_lh) + k_beta_log",
+                 "beta_fit": "k_gather_exp + k_ls_build + k_ge_lu + k_ge_subst (or k_nnls_lh) + k_beta_log",
                  "compacted_softmax": "k_ls_softmax", "normal_equations": "k_ls_build",
                  "lu_factorization": "k_ge_lu<false, true> (steps 0-127) + k_ge_lu_tail (the rest)",
                  "substitution": "k_ge_subst",

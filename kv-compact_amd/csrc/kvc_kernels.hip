@@ -4434,515 +4434,6 @@ k_ge_lu_tail(Geom g, const ChunkDesc * __restrict__ chunks, const float * __rest
     }
 }
 
-// Forward substitution y = L^-1 P b (the reference's elimination of the
-// right-hand sides: row i receives the updates of steps 0..i-1 in order,
-// skipped pivots contribute nothing), then back substitution (math.h:540-556)
-// x[i] = (y[i] - sum_{r>i} U[i][r] x[r]) / U[i][i] with r ascending. One wave
-// per 64 right-hand sides, lane v owns column v. The first 128 solved rows
-// of each sweep move from LDS into registers and are then read through a
-// statically unrolled loop; the other rows' earlier results come from LDS.
-// Each row of L / U (and its right-hand-side value) is loaded one row ahead
-// into registers, so its global-memory latency overlaps the previous row.
-constexpr int BS_HIGH = 128;
-constexpr int BS_PAD = 128;   // the row buffer holds entry k at rowb[BS_PAD - shift + k]
-constexpr int BS_AHEAD = 8;   // backward rows in flight
-constexpr int BS_FAHEAD = 4;  // forward 4-row blocks in flight
-constexpr int BS_LQ = 6;      // forward: multipliers read ahead in the register part
-constexpr int BS_UQ = 6;      // backward: float4 of U read ahead in the register part
-
-// val -= rowp[t] * xsb[t][lane] for t = 0 .. n_terms-1, ascending and
-// sequential. Sums of DS_B terms or more run in batches of DS_B: the first
-// batch is read at term 0 and applies its first (n_terms % DS_B, else DS_B)
-// terms, each later batch starts where the previous one stopped, and every
-// batch is read while the one before it is applied (two register sets
-// used in turn; a batch past the end is read at the last in-range start
-// n_terms - DS_B and not applied, so no read leaves [0, n_terms) and the
-// reads need no branches around them). The scheduling fences keep the
-// reads ahead of the arithmetic, so the LDS latency overlaps a batch of
-// the chain.
-constexpr int DS_B = 16;
-// val - r[0] * x[0] - r[1] * x[1] - ... in order: the products first, then
-// the subtractions back to back (a subtraction issued right after the one
-// it depends on waits less than one separated from it by a product).
-template <int B>
-__device__ __forceinline__ float sub_products(float val, const float (&r)[B], const float (&x)[B]) {
-    float p[B];
-#pragma unroll
-    for (int u = 0; u < B; u++) p[u] = r[u] * x[u];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < B; u++) val = val - p[u];
-    __builtin_amdgcn_sched_barrier(0);
-    return val;
-}
-__device__ __forceinline__ void ds_load(float (&r)[DS_B], float (&x)[DS_B], const float * rowp,
-                                        const float (*xsb)[64], int t0, int lane) {
-#pragma unroll
-    for (int u = 0; u < DS_B; u++) { r[u] = rowp[t0 + u]; x[u] = xsb[t0 + u][lane]; }
-}
-// the same batch with rowp + t0 16-byte aligned (float4 reads of rowp)
-__device__ __forceinline__ void ds_load4(float (&r)[DS_B], float (&x)[DS_B], const float * rowp,
-                                         const float (*xsb)[64], int t0, int lane) {
-    const float4 * r4 = reinterpret_cast<const float4 *>(rowp + t0);
-#pragma unroll
-    for (int q = 0; q < DS_B / 4; q++) {
-        const float4 a = r4[q];
-        r[4 * q + 0] = a.x; r[4 * q + 1] = a.y; r[4 * q + 2] = a.z; r[4 * q + 3] = a.w;
-    }
-#pragma unroll
-    for (int u = 0; u < DS_B; u++) x[u] = xsb[t0 + u][lane];
-}
-__device__ __forceinline__ float dot_seq(float val, const float * rowp, const float (*xsb)[64], int n_terms,
-                                         int lane) {
-    if (n_terms < DS_B) {
-        float r[DS_B - 1], x[DS_B - 1];
-#pragma unroll
-        for (int u = 0; u < DS_B - 1; u++)
-            if (u < n_terms) { r[u] = rowp[u]; x[u] = xsb[u][lane]; }
-#pragma unroll
-        for (int u = 0; u < DS_B - 1; u++)
-            if (u < n_terms) val = val - r[u] * x[u];
-        return val;
-    }
-    const int rem = n_terms & (DS_B - 1);
-    const int first = rem ? rem : DS_B;
-    const int lastb = n_terms - DS_B;
-    float ra[DS_B], xa[DS_B], rb[DS_B], xb[DS_B];
-    ds_load(ra, xa, rowp, xsb, 0, lane);
-    int t = first;
-    ds_load(rb, xb, rowp, xsb, min(t, lastb), lane);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < DS_B; u++)
-        if (u < first) val = val - ra[u] * xa[u];
-    __builtin_amdgcn_sched_barrier(0);
-    while (t < n_terms) {
-        ds_load(ra, xa, rowp, xsb, min(t + DS_B, lastb), lane);
-        __builtin_amdgcn_sched_barrier(0);
-        val = sub_products(val, rb, xb);
-        t += DS_B;
-        if (t >= n_terms) break;
-        ds_load(rb, xb, rowp, xsb, min(t + DS_B, lastb), lane);
-        __builtin_amdgcn_sched_barrier(0);
-        val = sub_products(val, ra, xa);
-        t += DS_B;
-    }
-    return val;
-}
-
-// dot_seq for a number of terms n8 that is a multiple of 8, with rowp
-// 16-byte aligned: an odd eighth first, then batches of DS_B read one batch
-// ahead as in dot_seq (no partial batch, so no per-term selection).
-__device__ __forceinline__ float dot_seq8(float val, const float * rowp, const float (*xsb)[64], int n8,
-                                          int lane) {
-    if (n8 <= 0) return val;
-    const float4 * r4 = reinterpret_cast<const float4 *>(rowp);
-    float r8[8], x8[8];
-    if (n8 == 8) {
-        const float4 a = r4[0], b = r4[1];
-        r8[0] = a.x; r8[1] = a.y; r8[2] = a.z; r8[3] = a.w;
-        r8[4] = b.x; r8[5] = b.y; r8[6] = b.z; r8[7] = b.w;
-#pragma unroll
-        for (int u = 0; u < 8; u++) x8[u] = xsb[u][lane];
-        return sub_products(val, r8, x8);
-    }
-    float ra[DS_B], xa[DS_B], rb[DS_B], xb[DS_B];
-    int t;
-    if (n8 & 8) {
-        const float4 a = r4[0], b = r4[1];
-        r8[0] = a.x; r8[1] = a.y; r8[2] = a.z; r8[3] = a.w;
-        r8[4] = b.x; r8[5] = b.y; r8[6] = b.z; r8[7] = b.w;
-#pragma unroll
-        for (int u = 0; u < 8; u++) x8[u] = xsb[u][lane];
-        ds_load4(rb, xb, rowp, xsb, 8, lane);
-        __builtin_amdgcn_sched_barrier(0);
-        val = sub_products(val, r8, x8);
-        t = 8;
-    } else {
-        ds_load4(rb, xb, rowp, xsb, 0, lane);
-        t = 0;
-    }
-    const int lastb = n8 - DS_B;
-    while (true) {
-        ds_load4(ra, xa, rowp, xsb, min(t + DS_B, lastb), lane);
-        __builtin_amdgcn_sched_barrier(0);
-        val = sub_products(val, rb, xb);
-        t += DS_B;
-        if (t >= n8) break;
-        ds_load4(rb, xb, rowp, xsb, min(t + DS_B, lastb), lane);
-        __builtin_amdgcn_sched_barrier(0);
-        val = sub_products(val, ra, xa);
-        t += DS_B;
-        if (t >= n8) break;
-    }
-    return val;
-}
-
-// Four rows at once: val[t] -= lt[j][t] * xsb[j - j1][lane] for j = j1 .. j2-1,
-// each row's terms in ascending j (four independent sequential sums);
-// lt holds the four rows' entries interleaved (16 bytes per j). Batches of
-// D4_B steps, arranged and read ahead as in dot_seq.
-constexpr int D4_B = 8;
-__device__ __forceinline__ void d4_load(float4 (&l)[D4_B], float (&y)[D4_B], const float4 * lp,
-                                        const float (*xsb)[64], int t0, int lane) {
-#pragma unroll
-    for (int u = 0; u < D4_B; u++) { l[u] = lp[t0 + u]; y[u] = xsb[t0 + u][lane]; }
-}
-__device__ __forceinline__ void d4_apply(float (&val)[4], const float4 (&l)[D4_B], const float (&y)[D4_B], int cnt) {
-#pragma unroll
-    for (int u = 0; u < D4_B; u++) {
-        if (u < cnt) {
-            val[0] = val[0] - l[u].x * y[u];
-            val[1] = val[1] - l[u].y * y[u];
-            val[2] = val[2] - l[u].z * y[u];
-            val[3] = val[3] - l[u].w * y[u];
-        }
-    }
-}
-__device__ __forceinline__ void dot4_seq(float (&val)[4], const float4 * lt, const float (*xsb)[64], int j1, int j2,
-                                         int lane) {
-    const int n_terms = j2 - j1;
-    const float4 * lp = lt + j1;
-    if (n_terms < D4_B) {
-        float4 l[D4_B];
-        float y[D4_B];
-#pragma unroll
-        for (int u = 0; u < D4_B - 1; u++)
-            if (u < n_terms) { l[u] = lp[u]; y[u] = xsb[u][lane]; }
-        d4_apply(val, l, y, n_terms);
-        return;
-    }
-    const int rem = n_terms & (D4_B - 1);
-    const int first = rem ? rem : D4_B;
-    const int lastb = n_terms - D4_B;
-    float4 la[D4_B], lb[D4_B];
-    float ya[D4_B], yb[D4_B];
-    d4_load(la, ya, lp, xsb, 0, lane);
-    int t = first;
-    d4_load(lb, yb, lp, xsb, min(t, lastb), lane);
-    __builtin_amdgcn_sched_barrier(0);
-    d4_apply(val, la, ya, first);
-    __builtin_amdgcn_sched_barrier(0);
-    while (t < n_terms) {
-        d4_load(la, ya, lp, xsb, min(t + D4_B, lastb), lane);
-        __builtin_amdgcn_sched_barrier(0);
-        d4_apply(val, lb, yb, D4_B);
-        __builtin_amdgcn_sched_barrier(0);
-        t += D4_B;
-        if (t >= n_terms) break;
-        d4_load(lb, yb, lp, xsb, min(t + D4_B, lastb), lane);
-        __builtin_amdgcn_sched_barrier(0);
-        d4_apply(val, la, ya, D4_B);
-        __builtin_amdgcn_sched_barrier(0);
-        t += D4_B;
-    }
-}
-
-// the same sum without the terms of steps whose pivot was skipped (skp[t] == 0)
-__device__ __forceinline__ float dot_seq_skip(float val, const float * rowp, const float (*xsb)[64], int n_terms,
-                                              const float * skp, int lane) {
-    for (int t = 0; t < n_terms; t++)
-        if (skp[t] != 0.0f) val = val - rowp[t] * xsb[t][lane];
-    return val;
-}
-
-__global__ void __launch_bounds__(64)
-k_ge_solve(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restrict__ aug,
-           const long long * __restrict__ aug_off, const int * __restrict__ perm_in,
-           const unsigned char * __restrict__ skip_in, const float * __restrict__ LU_all,
-           float * __restrict__ Yt_all, float * __restrict__ Cv, int only_skip) {
-    const int sysl = blockIdx.x;   // (layer, chunk, head)
-    const int h = sysl % g.H, c_idx = (sysl / g.H) % g.n_chunks, layer = sysl / (g.H * g.n_chunks);
-    const ChunkDesc c = chunks[c_idx];
-    const int n = c.tc, p = g.dv;
-    if (n > RG_ROWS || n < 1) return;
-    const int lane = threadIdx.x;
-    const int v = blockIdx.y * 64 + lane;
-    const bool act = v < p;
-    const int vc = act ? v : p - 1;   // in-range column for the loads of idle lanes
-    // by physical row: multipliers left of the row's pivot step, U from it on
-    const float * __restrict__ LU = LU_all + (long long)sysl * RG_ROWS * RG_ROWS;
-    const float * __restrict__ B = aug + aug_off[sysl] + (long long)n * n;   // row-major RHS [r][v]
-    float * Yt = Yt_all + (long long)sysl * RG_ROWS * g.dv;
-    float * x = Cv + (((long long)layer * g.H + h) * g.t_total + c.off) * g.dv;
-    __shared__ float xs[BS_HIGH][64];
-    // the forward's interleaved multipliers and the row buffers share LDS:
-    // rowb[0] holds the forward's rows when pivots were skipped, and the
-    // backward alternates U rows between rowb[0] and rowb[1]
-    __shared__ __align__(16) union {
-        float4 lt[RG_ROWS];
-        float rowb[2][BS_PAD + RG_ROWS];
-    } srows;
-    float * const rowb = srows.rowb[0];
-    __shared__ float skf[RG_ROWS];   // 1 where the step eliminated, 0 where it was skipped
-    __shared__ int permL[RG_ROWS];
-    __shared__ int any_skip;
-    if (lane == 0) any_skip = 0;
-    __builtin_amdgcn_wave_barrier();
-    for (int i = lane; i < RG_ROWS; i += 64) {
-        const int sk = (i < n) ? skip_in[(long long)sysl * g.tc_max + i] : 0;
-        skf[i] = sk ? 0.0f : 1.0f;
-        permL[i] = (i < n) ? perm_in[(long long)sysl * g.tc_max + i] : 0;
-        if (sk) any_skip = 1;
-    }
-    __builtin_amdgcn_wave_barrier();
-    const bool sk = any_skip != 0;
-    if (only_skip && !sk) return;         // k_ge_subst solved this system
-    const float * frow = rowb + BS_PAD;   // forward rows, unshifted
-    float4 * frow4 = reinterpret_cast<float4 *>(rowb + BS_PAD);
-
-    float4 pf;
-    float pb;
-    if (!sk) {
-        // ---- forward, four rows at a time (no skipped pivots): the rows'
-        // multipliers sit interleaved in LDS; earlier results come from LDS
-        // (rows below 128 until row 128, then from registers) and the four
-        // sums run side by side; the 4 x 4 triangle finishes them in order.
-        float4 * const lt = srows.lt;
-        float yr[BS_HIGH];
-        // rows and right-hand sides of the next BS_FAHEAD blocks in flight
-        float4 qf[BS_FAHEAD][4];
-        float qb[BS_FAHEAD][4];
-        auto fetch = [&](int i0, float4 (&f)[4], float (&bb)[4]) {
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int r = permL[(i0 + t < n) ? i0 + t : i0];
-                f[t] = reinterpret_cast<const float4 *>(LU + (unsigned)(r * RG_ROWS))[lane];
-                bb[t] = B[(unsigned)(r * p + vc)];
-            }
-        };
-#pragma unroll
-        for (int k = 0; k < BS_FAHEAD; k++)
-            if (4 * k < n) fetch(4 * k, qf[k], qb[k]);
-        for (int ib = 0; ib < n; ib += 4 * BS_FAHEAD) {
-#pragma unroll
-        for (int k = 0; k < BS_FAHEAD; k++) {
-            const int i0 = ib + 4 * k;
-            if (i0 >= n) break;
-            const int nr = min(4, n - i0);
-            lt[4 * lane + 0] = make_float4(qf[k][0].x, qf[k][1].x, qf[k][2].x, qf[k][3].x);
-            lt[4 * lane + 1] = make_float4(qf[k][0].y, qf[k][1].y, qf[k][2].y, qf[k][3].y);
-            lt[4 * lane + 2] = make_float4(qf[k][0].z, qf[k][1].z, qf[k][2].z, qf[k][3].z);
-            lt[4 * lane + 3] = make_float4(qf[k][0].w, qf[k][1].w, qf[k][2].w, qf[k][3].w);
-            float val[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) val[t] = act ? qb[k][t] : 0.0f;
-            fetch(min(i0 + 4 * BS_FAHEAD, n - 1), qf[k], qb[k]);   // unconditional, as in the backward ring
-            __builtin_amdgcn_wave_barrier();
-            if (i0 <= BS_HIGH) {
-                dot4_seq(val, lt, xs, 0, i0, lane);
-            } else {
-                // entries read BS_LQ steps ahead of their use
-                float4 lq[BS_HIGH];
-#pragma unroll
-                for (int j = 0; j < BS_LQ; j++) lq[j] = lt[j];
-#pragma unroll
-                for (int j = 0; j < BS_HIGH; j++) {
-                    if (j + BS_LQ < BS_HIGH) lq[j + BS_LQ] = lt[j + BS_LQ];
-                    __builtin_amdgcn_sched_barrier(0);
-                    val[0] = val[0] - lq[j].x * yr[j];
-                    val[1] = val[1] - lq[j].y * yr[j];
-                    val[2] = val[2] - lq[j].z * yr[j];
-                    val[3] = val[3] - lq[j].w * yr[j];
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                dot4_seq(val, lt + BS_HIGH, xs, 0, i0 - BS_HIGH, lane);
-            }
-            // the block's own triangle, row by row
-            float yn[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (q < t) val[t] = val[t] - reinterpret_cast<const float *>(&lt[i0 + q])[t] * yn[q];
-                yn[t] = val[t];
-            }
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                if (t >= nr) break;
-                const int i = i0 + t;
-                xs[i < BS_HIGH ? i : i - BS_HIGH][lane] = yn[t];
-                if (act) Yt[(unsigned)(i * g.dv + v)] = yn[t];
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (i0 + 4 == BS_HIGH && n > BS_HIGH) {
-#pragma unroll
-                for (int j = 0; j < BS_HIGH; j++) yr[j] = xs[j][lane];
-                __builtin_amdgcn_wave_barrier();
-            }
-        }
-        }
-    } else {
-    // ---- forward: rows [0, lb) from LDS, then rows [lb, n) with [0, lb) in registers
-    const int lb = n < BS_HIGH ? n : BS_HIGH;
-    pf = reinterpret_cast<const float4 *>(LU + (unsigned)(permL[0] * RG_ROWS))[lane];
-    pb = B[(unsigned)(permL[0] * p + vc)];
-    for (int i = 0; i < lb; i++) {
-        frow4[lane] = pf;
-        float val = act ? pb : 0.0f;
-        if (i + 1 < n) {
-            const int rn = permL[i + 1];
-            pf = reinterpret_cast<const float4 *>(LU + (unsigned)(rn * RG_ROWS))[lane];
-            pb = B[(unsigned)(rn * p + vc)];
-        }
-        __builtin_amdgcn_wave_barrier();
-        val = sk ? dot_seq_skip(val, frow, xs, i, skf, lane) : dot_seq(val, frow, xs, i, lane);
-        xs[i][lane] = val;
-        if (act) Yt[(unsigned)(i * g.dv + v)] = val;
-        __builtin_amdgcn_wave_barrier();
-    }
-    if (n > BS_HIGH) {
-        float yr[BS_HIGH];
-#pragma unroll
-        for (int j = 0; j < BS_HIGH; j++) yr[j] = xs[j][lane];
-        for (int i = BS_HIGH; i < n; i++) {
-            frow4[lane] = pf;
-            float val = act ? pb : 0.0f;
-            if (i + 1 < n) {
-                const int rn = permL[i + 1];
-                pf = reinterpret_cast<const float4 *>(LU + (unsigned)(rn * RG_ROWS))[lane];
-                pb = B[(unsigned)(rn * p + vc)];
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (!sk) {
-#pragma unroll
-                for (int j = 0; j < BS_HIGH; j++) val -= frow[j] * yr[j];
-                val = dot_seq(val, frow + BS_HIGH, xs, i - BS_HIGH, lane);
-            } else {
-#pragma unroll
-                for (int j = 0; j < BS_HIGH; j++)
-                    if (skf[j] != 0.0f) val -= frow[j] * yr[j];
-                val = dot_seq_skip(val, frow + BS_HIGH, xs, i - BS_HIGH, skf + BS_HIGH, lane);
-            }
-            xs[i - BS_HIGH][lane] = val;
-            if (act) Yt[(unsigned)(i * g.dv + v)] = val;
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-    }
-
-    // ---- backward: rows [hb, n) first, then rows [0, hb) with [hb, n) in
-    // registers (xh). Rows run in groups of BS_AHEAD from the top of each
-    // part (n - hb is a multiple of BS_AHEAD), so a row's sum splits into
-    // the rows above it in its own group (kept in registers, w), the earlier
-    // groups of its part (from LDS, a multiple of 8 terms) and, below hb,
-    // the register part; each piece ascends, in that order. Row col of U
-    // sits at rowb[k & 1] + bsh (k = the row's place in its group), written
-    // while the row before it runs; bsh places the entries of the earlier
-    // groups (col0 + 1 on) 16-byte aligned and, when hb > 0, the register
-    // part's entries (hb on) too. U rows and y values are loaded BS_AHEAD
-    // rows ahead through a register ring.
-    const int hb = n > BS_HIGH ? n - BS_HIGH : 0;
-    const int bsh = BS_PAD - hb - (hb > 0 ? 0 : (n & 3));
-    float xh[BS_HIGH];
-    float w[BS_AHEAD];
-    float4 rf[BS_AHEAD];
-    float rb[BS_AHEAD];
-#pragma unroll
-    for (int k = 0; k < BS_AHEAD; k++) {
-        const int r = max(n - 1 - k, 0);
-        rf[k] = reinterpret_cast<const float4 *>(LU + (unsigned)(permL[r] * RG_ROWS))[lane];
-        rb[k] = Yt[(unsigned)(r * g.dv + vc)];
-    }
-    {
-        float * b0 = srows.rowb[0] + bsh;
-        b0[4 * lane + 0] = rf[0].x;
-        b0[4 * lane + 1] = rf[0].y;
-        b0[4 * lane + 2] = rf[0].z;
-        b0[4 * lane + 3] = rf[0].w;
-    }
-    for (int col0 = n - 1; col0 >= 0; col0 -= BS_AHEAD) {
-        const bool upper = col0 >= hb;            // the whole group is on one side of hb
-        const int xoff = upper ? hb : 0;           // row r's result sits at xs[r - xoff]
-        const int n8 = (upper ? n : hb) - col0 - 1;   // earlier groups of this part
-        // physical rows of the next group, lane k holding row col0 - BS_AHEAD - k
-        const int pnext = permL[max(col0 - BS_AHEAD - (lane & (BS_AHEAD - 1)), 0)];
-#pragma unroll
-        for (int k = 0; k < BS_AHEAD; k++) {
-            const int col = col0 - k;
-            if (col < 0) break;
-            if (col == hb - 1) {
-                // entering the rows below hb: rows [hb, n) move to registers
-#pragma unroll
-                for (int i = 0; i < BS_HIGH; i++) xh[i] = xs[i][lane];
-                __builtin_amdgcn_wave_barrier();
-            }
-            const float * brow = srows.rowb[k & 1] + bsh;
-            const float * bhi = srows.rowb[k & 1] + BS_PAD;   // == brow + hb when hb > 0
-            {
-                // the next row's U (ring slot k + 1) into the other buffer
-                float * bn = srows.rowb[(k + 1) & 1] + bsh;
-                const float4 f = rf[(k + 1) % BS_AHEAD];
-                bn[4 * lane + 0] = f.x;
-                bn[4 * lane + 1] = f.y;
-                bn[4 * lane + 2] = f.z;
-                bn[4 * lane + 3] = f.w;
-            }
-            const float yv = rb[k];
-            const float piv = brow[col];
-            float ug[BS_AHEAD];   // U entries of the rows above col in the group
-#pragma unroll
-            for (int j = 0; j < k; j++) ug[j] = brow[col + 1 + j];
-            float val = g.zero_val;
-            if (!(fabsf(piv) < 1e-12f)) {
-                val = act ? yv : 0.0f;
-                if (k > 0) {
-                    float pg[BS_AHEAD];
-#pragma unroll
-                    for (int j = 0; j < k; j++) pg[j] = ug[j] * w[k - 1 - j];
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int j = 0; j < k; j++) val = val - pg[j];
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                val = dot_seq8(val, brow + col0 + 1, xs + (col0 + 1 - xoff), n8, lane);
-                if (!upper) {
-                    // U entries read BS_UQ float4 ahead of their use
-                    const float4 * bhi4 = reinterpret_cast<const float4 *>(bhi);
-                    float4 uq[BS_HIGH / 4];
-#pragma unroll
-                    for (int q = 0; q < BS_UQ; q++) uq[q] = bhi4[q];
-#pragma unroll
-                    for (int q = 0; q < BS_HIGH / 4; q += 2) {
-                        if (q + BS_UQ < BS_HIGH / 4) uq[q + BS_UQ] = bhi4[q + BS_UQ];
-                        if (q + 1 + BS_UQ < BS_HIGH / 4) uq[q + 1 + BS_UQ] = bhi4[q + 1 + BS_UQ];
-                        __builtin_amdgcn_sched_barrier(0);
-                        const float r8[8] = {uq[q].x, uq[q].y, uq[q].z, uq[q].w,
-                                             uq[q + 1].x, uq[q + 1].y, uq[q + 1].z, uq[q + 1].w};
-                        const float x8[8] = {xh[4 * q + 0], xh[4 * q + 1], xh[4 * q + 2], xh[4 * q + 3],
-                                             xh[4 * q + 4], xh[4 * q + 5], xh[4 * q + 6], xh[4 * q + 7]};
-                        val = sub_products(val, r8, x8);
-                    }
-                }
-                val = val / piv;
-            }
-            w[k] = val;
-            xs[col - xoff][lane] = val;
-            {
-                // the slot's next row, refilled once its values are dead and
-                // unconditionally (row 0 again near the end): otherwise the
-                // slot holds two live values, and the copy that merges them
-                // waits for every load in flight
-                const int r = max(col - BS_AHEAD, 0);
-                const int pr = __builtin_amdgcn_readlane(pnext, k);
-                rf[k] = reinterpret_cast<const float4 *>(LU + (unsigned)(pr * RG_ROWS))[lane];
-                rb[k] = Yt[(unsigned)(r * g.dv + vc)];
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-    // the solution goes out after the sweep (stores inside it would make
-    // the waits for the row loads drain every access in flight): rows
-    // [0, hb) from LDS, rows [hb, n) from registers when n > BS_HIGH
-    if (act) {
-        for (int i = 0; i < (hb > 0 ? hb : n); i++) x[(unsigned)(i * g.dv + v)] = xs[i][lane];
-        if (hb > 0) {
-#pragma unroll
-            for (int i = 0; i < BS_HIGH; i++) x[(unsigned)((hb + i) * g.dv + v)] = xh[i];
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Forward and back substitution of the register-LU systems (n <= 256). The
 // forward pass is the reference's elimination of the right-hand-side columns
@@ -5723,9 +5214,10 @@ k_ge_subst_wide(Geom g, const ChunkDesc * __restrict__ chunks, const float * __r
 
 // The systems with skipped steps, usually none or a few of many: every block
 // looks through its share of the systems (x, x + gridDim.x, ..) eight at a
-// time, then solves the ones it found. k_ge_solve, which took them one wave
-// per 64 columns before, held a call up for 1.77 ms per such system (256
-// unknowns), 0.3 ms here. grid (blocks, ceil(p / 64)).
+// time, then solves the ones it found. One wave per 64 columns, reading rows
+// back from LDS, held a call up for 1.77 ms per such system (256 unknowns),
+// 0.3 ms here; a clamped fit of 3328 systems, all of them singular: 16.6 ms a
+// call that way, 13.8 this. grid (blocks, ceil(p / 64)).
 constexpr int SW_LIST = 256;
 
 __global__ void __launch_bounds__(64 * SW_WAVES)
@@ -7903,44 +7395,33 @@ static bool subst_wide_enabled() {
 }
 
 void launch_ge_solve(const Geom & g, const Work & w, float * Cv, hipStream_t st) {
-    const unsigned systems = (unsigned)(g.L * g.n_chunks * g.H);
-    // k_ge_subst or k_ge_subst_wide solves every system without a skipped pivot
-    // step, k_ge_subst_skip the others (KVC_SOLVE_OLD=1, or without the LDS:
-    // k_ge_solve)
-    static const bool old_solve = [] {
-        const char * e = getenv("KVC_SOLVE_OLD");
-        return e && e[0] == '1';
-    }();
-    // k_ge_subst_wide runs one block per CU: 288 us for 256 unknowns as long as
-    // every block has its CU, 580 us for 320 of them, where k_ge_subst (eight
-    // waves per CU) still takes 420 us
-    static const bool wide_ok = hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst_wide),
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                    SW_LDS * (int)sizeof(float)) == hipSuccess &&
-                                hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst_skip),
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                    SW_LDS * (int)sizeof(float)) == hipSuccess;
-    if (!old_solve && wide_ok && subst_wide_enabled() && (long long)systems * cdiv(g.dv, 64) <= SW_MAX_BLOCKS) {
-        hipLaunchKernelGGL(k_ge_subst_wide, dim3(systems, cdiv(g.dv, 64)), dim3(64 * SW_WAVES),
-                           SW_LDS * sizeof(float), st, g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv);
-    } else if (!old_solve) {
-        const unsigned nw = cdiv(g.dv, 64);
-        const size_t lds = (size_t)nw * SB_LROWS * 64 * sizeof(float);
-        static int lds_ok = -1;
-        if (lds_ok < 0)
-            lds_ok = hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         4 * SB_LROWS * 64 * (int)sizeof(float)) == hipSuccess;
-        hipLaunchKernelGGL(k_ge_subst, dim3(systems), dim3(64 * nw), lds, st,
-                           g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, Cv);
-    }
-    if (!old_solve && wide_ok)
-        hipLaunchKernelGGL(k_ge_subst_skip, dim3(std::min(systems, 256u), cdiv(g.dv, 64)), dim3(64 * SW_WAVES),
-                           SW_LDS * sizeof(float), st, g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv,
-                           (int)systems);
+    const unsigned systems = (unsigned)(g.L * g.n_chunks * g.H), nw = cdiv(g.dv, 64);
+    // dynamic LDS beyond 64 KB needs the kernel attribute (once per process);
+    // without it the launch fails, and run_batch's error check returns -6
+    static const bool lds_ok = hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst_wide),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   SW_LDS * (int)sizeof(float)) == hipSuccess &&
+                               hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst_skip),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   SW_LDS * (int)sizeof(float)) == hipSuccess &&
+                               hipFuncSetAttribute(reinterpret_cast<const void *>(k_ge_subst),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   4 * SB_LROWS * 64 * (int)sizeof(float)) == hipSuccess;
+    (void)lds_ok;
+    // k_ge_subst or k_ge_subst_wide solves every system without a skipped
+    // pivot step, k_ge_subst_skip the others. k_ge_subst_wide runs one block
+    // per CU: 288 us for 256 unknowns as long as every block has its CU, 580
+    // us for 320 of them, where k_ge_subst (eight waves per CU) still takes
+    // 420 us
+    if (subst_wide_enabled() && (long long)systems * nw <= SW_MAX_BLOCKS)
+        hipLaunchKernelGGL(k_ge_subst_wide, dim3(systems, nw), dim3(64 * SW_WAVES), SW_LDS * sizeof(float), st,
+                           g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv);
     else
-        hipLaunchKernelGGL(k_ge_solve, dim3(systems, cdiv(g.dv, 64)), dim3(64), 0, st,
-                           g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv, old_solve ? 0 : 1);
+        hipLaunchKernelGGL(k_ge_subst, dim3(systems), dim3(64 * nw), (size_t)nw * SB_LROWS * 64 * sizeof(float), st,
+                           g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, Cv);
+    hipLaunchKernelGGL(k_ge_subst_skip, dim3(std::min(systems, 256u), nw), dim3(64 * SW_WAVES),
+                       SW_LDS * sizeof(float), st, g, w.chunks, w.aug, w.aug_off, w.perm, w.skip, w.LU, w.Bt, Cv,
+                       (int)systems);
     if (g.tc_max > RG_ROWS) {
         // dynamic LDS: the largest system's panels (3 pb n floats), or the
         // step-by-step factors; the attribute once per process
