@@ -7138,7 +7138,7 @@ void launch_chunk_softmax(const Geom & g, const Work & w, hipStream_t st) {
                            g, w.chunks, g.score_method != 0 ? w.amax : w.imp, w.sens);
 }
 
-constexpr long long RT_NARROW = 320, RT_WIDE = 1024;
+constexpr long long RT_NARROW = 192, RT_NARROW_32 = 320, RT_WIDE = 1024;
 constexpr unsigned RT_SPARE_LDS = 11 * 1024;
 
 template <int VC>
@@ -7149,13 +7149,19 @@ void launch_refit_inst(const Geom & g, const Work & w, const float * V, bool ali
     };
     // Column blocks as wide as d_v allows. Queries 64 at a time (a 64- or
     // 32-column block then gives a thread 4 or 2 x 4 sums) where that still
-    // leaves RT_WIDE blocks, else 32. Below RT_NARROW blocks of 32 queries a
-    // block's chain over the keys is what is waited for, and one sum per
-    // thread is faster.
+    // leaves RT_WIDE blocks, else 32 (64 columns, 512-key chunks: 512 blocks
+    // 61 us against 64, 1024 blocks 112 against 123, 256 blocks 50 against 36).
+    // Below RT_NARROW blocks of 32 queries a block's chain over the keys is
+    // what is waited for, and one sum per thread is faster. 1280-key chunks,
+    // narrow against tiles: 128 columns 42 / 105 us at 64 blocks, 85 / 110 at
+    // 128, 116 / 116 at 192, 158 / 120 at 256; 64 columns 61 / 69 at 192,
+    // 87 / 70 at 256; 32 columns 34 / 47 at 192, 62 / 60 at 384. Against the
+    // kernel for any width (40 columns 102 / 471 at 384, 188 / 505 at 768) the
+    // line could lie higher still.
     const long long units = (long long)grid.x * grid.y;
     const int vb = g.dv % 128 == 0 ? 128 : (g.dv % 64 == 0 ? 64 : (g.dv % 32 == 0 ? 32 : 0));
     const unsigned q32 = cdiv(g.nq_max, 32), q64 = cdiv(g.nq_max, 64);
-    if (units * q32 * (vb ? g.dv / vb : 1) < RT_NARROW) {
+    if (units * q32 * (vb ? g.dv / vb : 1) < (aligned && vb >= 64 ? RT_NARROW : RT_NARROW_32)) {
         go(k_refit_target_narrow<VC>, cdiv(g.nq_max, RN_QB) * cdiv(g.dv, RN_VB));
     } else if (!aligned || vb == 0) {
         go(k_refit_target_any<VC>, q32);
@@ -7165,7 +7171,8 @@ void launch_refit_inst(const Geom & g, const Work & w, const float * V, bool ali
         // it needs to finish with it (100k tokens, 32 layers: the Gram 8.8 ms
         // at five, 10.4 at seven, the refit target 11.4 and 10.1)
         // (a unit's query blocks in one block, its values still in L2, where the
-        // units alone fill the chip)
+        // units alone fill the chip: 64 queries, 2048 units 1006 us against 1044,
+        // 512 units 281 against 263, within 4% either way up to 4096)
         const unsigned nv = g.dv / 128;
         go(k_refit_target<VC, 128, 32>, (units * nv >= 2048 ? 1 : q32) * nv, RT_SPARE_LDS);
     } else {

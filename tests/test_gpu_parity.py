@@ -302,7 +302,8 @@ def test_many_reference_queries(gpu, orc):
 @pytest.mark.parametrize("T,H,d,nq,chunk", [
     (300, 1, 32, 1, -1), (300, 2, 40, 17, -1), (257, 1, 256, 33, -1), (130, 4, 64, 64, -1), (65, 1, 128, 65, -1),
     (5135, 8, 128, 33, 128), (5135, 8, 64, 33, 128), (5135, 8, 32, 20, 128), (5135, 8, 96, 33, 128),
-    (5135, 8, 40, 33, 128), (2600, 8, 256, 20, 128), (16500, 8, 64, 65, 128), (8230, 8, 96, 65, 128)])
+    (5135, 8, 40, 33, 128), (3300, 8, 128, 20, 128), (3300, 8, 32, 20, 128),
+    (2600, 8, 256, 20, 128), (16500, 8, 64, 65, 128), (8230, 8, 96, 65, 128)])
 def test_refit_target_blocks(gpu, orc, T, H, d, nq, chunk):
     print(f"[refit] T={T} H={H} d={d} nq={nq} chunk={chunk}", flush=True)
     K, V = kv_cache(T, H, d, 53, channel_scale=True)
