@@ -1067,8 +1067,8 @@ k_refit_target_narrow(Geom g, const ChunkDesc * __restrict__ chunks, const float
     const int n = c.Tc, tid = threadIdx.x, tq = tid >> 4, tv = tid & 15;
     // loaders, four elements each at clamped positions: weights, thread ->
     // query (tid >> 6) + 4 u, key tid & 63; values, thread -> key
-    // (tid >> 4) + 16 u, column tid & 15. Keys past n get weight 0 and the
-    // last key's value times 0 is not used: the sum stops at n.
+    // (tid >> 4) + 16 u, column tid & 15. Positions past n hold key n - 1's
+    // again and are not summed.
     const int kk = tid & 63, cc = min(v0 + tv, g.dv - 1);
     const float * ar[4];
     float sc[4], ra[4], rv[4];
@@ -7110,6 +7110,14 @@ void launch_scores(const Geom & g, const ChunkDesc * chunks, int n_chunk_units, 
     }
 }
 
+// Units from which one block takes a unit's rows, exponentials and importance.
+// 1280 keys, one block a unit against rows and keys over the grid (8 or 32
+// rows a block): 64 queries 119 / 67 / 77 us at 256 units, 154 / 105 / 100 at
+// 384, 194 / 194 / 168 at 768, 236 / 262 / 240 at 1024, 450 / 514 / 448 at
+// 2048; 32 queries 70 / 55 / 66 at 384, 79 / 68 / 74 at 512, 98 / 102 / 95 at
+// 768, 116 / 130 / 119 at 1024. The sides meet at 800 to 1000 units; 512 is on
+// the safe side of that, and so is the inner line of 512 blocks of 32 rows
+// (between 256 and 384 units of 64 queries they are level).
 constexpr long long SM_UNITS = 512;
 
 void launch_chunk_softmax(const Geom & g, const Work & w, hipStream_t st) {
@@ -7349,10 +7357,17 @@ void launch_ls_build(const Geom & g, const Work & w, hipStream_t st, bool m_by_l
                            st, g, w.chunks, w.X, w.Y, w.aug, w.aug_off, lds_floats, m_by_lu ? 1 : 0);
         return;
     }
-    // the most tiles per thread that leave two blocks per CU (four, at three
-    // waves per SIMD, only with rows enough to sum: 32 rows of 256 + 256
-    // columns took 1.67 ms with two, 2.03 ms with four); a block takes several
-    // passes only where the systems alone give the GPU 2048 blocks
+    // the most tiles per thread that leave two blocks per CU (256 + 128
+    // columns, 64 rows: 64 systems 25 us with one, 26 with two, 44 with four;
+    // 128 systems 44, 36, 49; 256 systems 78, 66, 63). Four, at three waves per
+    // SIMD, only with rows enough to sum (32 rows of 256 + 256 columns: 1.67 ms
+    // with two, 2.03 with four). They read X less often, which pays on long
+    // contexts, whose rows of X lie far apart (26 chunks a layer, 6656 systems:
+    // 2.73 ms with four, 2.94 with two, the call 21.4 and 22.0), and costs on
+    // short ones with few tiles (4 chunks, 4096 systems: 1.14 ms with four,
+    // 0.98 with two; 64 columns of Y 0.62 and 0.49); the long ones were
+    // preferred. A block takes several passes only where the systems alone
+    // give the GPU 2048 blocks
     const long long systems = (long long)g.n_chunks * g.H * g.L;
     const int nbi = cdiv(g.tc_max, 4), nbw = wmax / 4;
     const bool skip_m = m_by_lu && g.tc_max <= 256;
