@@ -2676,8 +2676,11 @@ k_beta_log(float * __restrict__ wb, long long n) {
 //   * The gradient's terms with w == 0 are left out (x + 0 = x): only where
 //     every entry of AtA is finite, which its diagonal shows.
 // The 10-layer, 16-chunk, 4-head fit at n = 256 with 32 queries: 79.9 ms with
-// the sub-problem in LDS and all 200 passes, 1.6 ms now (two waves on every
-// system: 2.7 ms). 64 queries, 8 chunks: the whole call 128 -> 16.4 ms.
+// the sub-problem in LDS and all 200 passes, 1.9 ms now (two waves on every
+// system: 2.8 ms). With 64 queries, every system on two waves, 12 to 22 ms; the
+// whole call with one refinement round 452 -> 37 ms (SnapKV's 64) and 514 -> 50
+// (the library's own). A resident wave issues a VALU instruction every 13
+// clocks and waits 0.40 to 0.44 of its time.
 // ---------------------------------------------------------------------------
 constexpr int LH_PMAX = 128;   // passive-set capacity
 constexpr int LH_SB = 4;       // elimination steps per rotation of the registers
@@ -4900,9 +4903,12 @@ k_ge_subst(Geom g, const ChunkDesc * __restrict__ chunks, const float * __restri
 // per (system, 64 columns) instead of one, lane = column throughout. One wave
 // alone issues an instruction every 4.4 cycles, so the 65,000 terms of a
 // 256-unknown column take k_ge_subst 420 us however few systems there are
-// (128 unknowns 219 us); here 288 and 104 us, of which the forward pass is 55
-// and 21 us and the rest the backward chain, 11 cycles per subtraction
-// whether its products come from LDS or from registers.
+// (128 unknowns 219 us); here 290 and 106 us, of which the forward pass is 55
+// and 21 us and the rest the backward chain: by these two sizes about 10
+// cycles per subtraction (0.55 of it at 256 unknowns; the same whether the
+// products come from LDS or from registers, 5.8 for subtractions back to back
+// and alone) and 970 per row for the barrier, the first LDS reads after it, the
+// division and the result's way to the helpers.
 //   Forward: wave w owns row groups w, w + 8, .. (eight rows each) in
 // registers. When a group is finished its rows go to LDS and every wave takes
 // their eight steps off its later rows; the next group's owner does that group
@@ -7174,10 +7180,11 @@ void launch_refit_inst(const Geom & g, const Work & w, const float * V, bool ali
     } else if (!aligned || vb == 0) {
         go(k_refit_target_any<VC>, q32);
     } else if (vb == 128) {
-        // five blocks per CU (the unused LDS; its registers would allow seven):
-        // with more, the diversity Gram beside it gets less of the chip than
-        // it needs to finish with it (100k tokens, 32 layers: the Gram 8.8 ms
-        // at five, 10.4 at seven, the refit target 11.4 and 10.1)
+        // (97 registers: four blocks per CU. The unused LDS leaves a CU less
+        // room for the diversity Gram's blocks beside four of these, and both
+        // end a little sooner: 100k tokens, 32 layers, the Gram 7.6-7.8 ms
+        // against 8.1-8.3, the refit target 11.2-11.3 against 11.3-11.4; the
+        // call is the same within 0.3%.)
         // (a unit's query blocks in one block, its values still in L2, where the
         // units alone fill the chip: 64 queries, 2048 units 1006 us against 1044,
         // 512 units 281 against 263, within 4% either way up to 4096)
@@ -7294,7 +7301,7 @@ void launch_nnls_lh(const Geom & g, const Work & w, float * wout, int max_iter, 
     const dim3 grid(g.n_chunks * g.H, g.L);
     // passive sets outgrow the query count by one or two variables, seldom
     // more (rank and rounding), so up to 62 queries the one-wave instance goes
-    // first (32 queries, 640 systems of 256: 1.6 ms against 2.7 ms on two
+    // first (32 queries, 640 systems of 256: 1.9 ms against 2.8 ms on two
     // waves) and the other takes what it left
     int * redo = g.nq_max <= 62 ? w.lu_redo : nullptr;
     if (redo)

@@ -42,9 +42,10 @@ def weights(model, waves, first, M, b, cap):
     """The kernel's weights, clamped as k_beta_log does, and its redo flag."""
     n = M.shape[1]
     ata, atb = np.zeros((n, n), np.float32), np.zeros(n, np.float32)
-    for q in range(M.shape[0]):   # sums in row order, as k_ls_build's
-        ata = ata + M[q][:, None] * M[q][None, :]
-        atb = atb + M[q] * b[q]
+    with np.errstate(over="ignore"):
+        for q in range(M.shape[0]):   # sums in row order, as k_ls_build's
+            ata = ata + M[q][:, None] * M[q][None, :]
+            atb = atb + M[q] * b[q]
     r = subprocess.run([str(model)], input=struct.pack("<4i", waves, first, n, cap) + ata.tobytes() + atb.tobytes(),
                        capture_output=True, timeout=300)
     assert r.returncode == 0, r.stderr.decode()[-3000:]
